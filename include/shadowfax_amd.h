@@ -33,7 +33,7 @@ extern "C" {
 #define SFX_HLLC 1
 
 /* precision variants */
-#define SFX_PREC_FP64 0  /* plain FP64, reference association (parity path) */
+#define SFX_PREC_FP64 0  /* FP64, the reference's expressions and iteration (parity path) */
 #define SFX_PREC_MIXED 1 /* FP32 bulk, FP64 final Newton step for p*, FP64
                             conserved-quantity accumulation */
 

@@ -154,8 +154,9 @@ __global__ __launch_bounds__(256) void drain_gradients(flux::MeshView<T> m, T* _
     });
 }
 
-template <int ND, int KIND, int MIXED, typename T, typename R>
-__global__ __launch_bounds__(256) void drain_faces(flux::MeshView<T> m, const T* __restrict__ grad,
+template <int ND, int KIND, int MIXED, typename T, typename R, int ROOT>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(flux::face_waves<ND, KIND, MIXED>(), 10))) void drain_faces(flux::MeshView<T> m, const T* __restrict__ grad,
                                                    Consts cd, mixed::CF cf,
                                                    T* __restrict__ dQL,
                                                    uint8_t* __restrict__ fstatus,
@@ -163,8 +164,8 @@ __global__ __launch_bounds__(256) void drain_faces(flux::MeshView<T> m, const T*
                                                    Plan* __restrict__ p, int grid) {
     unsigned cnt[CNT_N] = {0u, 0u, 0u, 0u, 0u};
     drain<true>(p, 1, grid, [&](const Slot& sl, int64_t f) {
-        flux::face_item<ND, KIND, MIXED, T, R>(m, f, grad, sl.gshift, cd, cf, dQL, sl.qshift,
-                                               fstatus, cnt);
+        flux::face_item<ND, KIND, MIXED, T, R, false, ROOT>(m, f, grad, sl.gshift, cd, cf, dQL,
+                                                            sl.qshift, fstatus, cnt);
     });
     block_add_counters(ctr, cnt);
 }
@@ -209,8 +210,9 @@ __global__ __launch_bounds__(256) void range_gradients(flux::MeshView<T> m, T* _
     if(k < ncell) flux::grad_cell<ND, T, R, DIFF>(m, cell0 + k, grad, gshift);
 }
 
-template <int ND, int KIND, int MIXED, typename T, typename R>
-__global__ __launch_bounds__(256) void range_faces(flux::MeshView<T> m, const T* __restrict__ grad,
+template <int ND, int KIND, int MIXED, typename T, typename R, int ROOT>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(flux::face_waves<ND, KIND, MIXED>(), 10))) void range_faces(flux::MeshView<T> m, const T* __restrict__ grad,
                                                    Consts cd, mixed::CF cf,
                                                    T* __restrict__ dQL,
                                                    uint8_t* __restrict__ fstatus,
@@ -220,8 +222,8 @@ __global__ __launch_bounds__(256) void range_faces(flux::MeshView<T> m, const T*
     const int64_t k = xcd_block() * blockDim.x + threadIdx.x;
     unsigned cnt[CNT_N] = {0u, 0u, 0u, 0u, 0u};
     if(k < nface)
-        flux::face_item<ND, KIND, MIXED, T, R>(m, face0 + k, grad, gshift, cd, cf, dQL, qshift,
-                                               fstatus, cnt);
+        flux::face_item<ND, KIND, MIXED, T, R, false, ROOT>(m, face0 + k, grad, gshift, cd, cf, dQL,
+                                                            qshift, fstatus, cnt);
     block_add_counters(ctr, cnt);
 }
 

@@ -25,11 +25,15 @@ hipError_t ens_step_impl(int ndim, int kind, const EnsArgs<T>& a, hipStream_t s)
         hipLaunchKernelGGL((ens::drain_gradients<ND, T, double, MIXED != 0>), gc, b, 0, s, a.m, \
                            a.grad, a.plan, grid);                                               \
         if(kind == 0)                                                                          \
-            hipLaunchKernelGGL((ens::drain_faces<ND, 0, MIXED, T, double>), gf, b, 0, s, a.m,   \
-                               a.grad, a.c, cf, a.dQL, a.fstatus, a.ctr, a.plan, grid);         \
+            with_root<MIXED == 0>(a.c, [&](auto root) {                                        \
+                hipLaunchKernelGGL((ens::drain_faces<ND, 0, MIXED, T, double,                  \
+                                                     decltype(root)::value>),                  \
+                                   gf, b, 0, s, a.m, a.grad, a.c, cf, a.dQL, a.fstatus, a.ctr, \
+                                   a.plan, grid);                                              \
+            });                                                                                \
         else                                                                                   \
-            hipLaunchKernelGGL((ens::drain_faces<ND, 1, MIXED, T, double>), gf, b, 0, s, a.m,   \
-                               a.grad, a.c, cf, a.dQL, a.fstatus, a.ctr, a.plan, grid);         \
+            hipLaunchKernelGGL((ens::drain_faces<ND, 1, MIXED, T, double, 0>), gf, b, 0, s,     \
+                               a.m, a.grad, a.c, cf, a.dQL, a.fstatus, a.ctr, a.plan, grid);    \
         hipLaunchKernelGGL((ens::drain_gather<ND, MIXED, T>), gc, b, 0, s, a.m.gather_off,         \
                            a.m.gather_entry, a.m.ghost, a.m.twin, a.dQL, a.dQ, a.plan, grid);   \
         hipLaunchKernelGGL((ens::drain_update<ND>), gc, b, 0, s, a.c, a.Q, a.dQ, a.m.volume,    \
@@ -57,11 +61,14 @@ hipError_t ens_range_impl(int ndim, int kind, const EnsArgs<T>& a, int64_t cell0
                            a.grad, cell0, ncell, gshift);                                       \
         if(nface > 0) {                                                                        \
             if(kind == 0)                                                                      \
-                hipLaunchKernelGGL((ens::range_faces<ND, 0, MIXED, T, double>), gf, b, 0, s,    \
-                                   a.m, a.grad, a.c, cf, a.dQL, a.fstatus, a.ctr, face0,        \
-                                   nface, gshift, qshift);                                      \
+                with_root<MIXED == 0>(a.c, [&](auto root) {                                    \
+                    hipLaunchKernelGGL((ens::range_faces<ND, 0, MIXED, T, double,              \
+                                                         decltype(root)::value>),              \
+                                       gf, b, 0, s, a.m, a.grad, a.c, cf, a.dQL, a.fstatus,    \
+                                       a.ctr, face0, nface, gshift, qshift);                   \
+                });                                                                            \
             else                                                                               \
-                hipLaunchKernelGGL((ens::range_faces<ND, 1, MIXED, T, double>), gf, b, 0, s,    \
+                hipLaunchKernelGGL((ens::range_faces<ND, 1, MIXED, T, double, 0>), gf, b, 0, s, \
                                    a.m, a.grad, a.c, cf, a.dQL, a.fstatus, a.ctr, face0,        \
                                    nface, gshift, qshift);                                      \
         }                                                                                      \
@@ -84,12 +91,15 @@ hipError_t ens_queue_impl(int ndim, int kind, const EnsArgs<T>& a, const QueueAr
                           hipStream_t s, int* blocks) {
     mixed::CF cf = mixed::make_cf(a.c);
     const void* fn = nullptr;
-    if(ndim == 3)
-        fn = kind == 0 ? (const void*)ens::queue_kernel<3, 0, MIXED, T, double>
-                       : (const void*)ens::queue_kernel<3, 1, MIXED, T, double>;
+    if(kind != 0)
+        fn = ndim == 3 ? (const void*)ens::queue_kernel<3, 1, MIXED, T, double, 0>
+                       : (const void*)ens::queue_kernel<2, 1, MIXED, T, double, 0>;
     else
-        fn = kind == 0 ? (const void*)ens::queue_kernel<2, 0, MIXED, T, double>
-                       : (const void*)ens::queue_kernel<2, 1, MIXED, T, double>;
+        with_root<MIXED == 0>(a.c, [&](auto root) {
+            constexpr int ROOT = decltype(root)::value;
+            fn = ndim == 3 ? (const void*)ens::queue_kernel<3, 0, MIXED, T, double, ROOT>
+                           : (const void*)ens::queue_kernel<2, 0, MIXED, T, double, ROOT>;
+        });
     const size_t shmem = 4 * (size_t)qa.nmesh_words;
     int per_cu = 0;
     hipError_t err = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, a.block, shmem);

@@ -267,11 +267,11 @@ __device__ __forceinline__ void q_gradients(const EnsArgs<T>& a) {
         flux::grad_cell<ND, T, R, DIFF>(a.m, i, a.grad, sl.gshift);
     });
 }
-template <int ND, int KIND, int MIXED, typename T, typename R>
+template <int ND, int KIND, int MIXED, typename T, typename R, int ROOT>
 __device__ __forceinline__ void q_faces(const EnsArgs<T>& a, const mixed::CF& cf,
                                      unsigned (&cnt)[CNT_N]) {
     drain<true>(a.plan, 1, 0, [&](const Slot& sl, int64_t f) {
-        flux::face_item<ND, KIND, MIXED, T, R>(a.m, f, a.grad, sl.gshift, a.c, cf, a.dQL,
+        flux::face_item<ND, KIND, MIXED, T, R, false, ROOT>(a.m, f, a.grad, sl.gshift, a.c, cf, a.dQL,
                                                sl.qshift, a.fstatus, cnt);
     });
 }
@@ -302,7 +302,7 @@ constexpr int queue_waves() {
     return ND == 2 ? SFX_QUEUE_WAVES_2D : 2;
 }
 
-template <int ND, int KIND, int MIXED, typename T, typename R>
+template <int ND, int KIND, int MIXED, typename T, typename R, int ROOT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(queue_waves<ND>()))) void
 queue_kernel(EnsArgs<T> a, mixed::CF cf, DevQueue* q,
                                                     HostBox* box, const int32_t* box_mesh,
@@ -325,7 +325,7 @@ queue_kernel(EnsArgs<T> a, mixed::CF cf, DevQueue* q,
         if(__hip_atomic_load(&q->stop, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT)) break;
         q_gradients<ND, T, R, MIXED != 0>(a);
         if(!grid_barrier(q, nb, gen)) break;
-        q_faces<ND, KIND, MIXED, T, R>(a, cf, cnt);
+        q_faces<ND, KIND, MIXED, T, R, ROOT>(a, cf, cnt);
         if(!grid_barrier(q, nb, gen)) break;
         q_gather<ND, MIXED, T>(a);
         if(!grid_barrier(q, nb, gen)) break;

@@ -54,14 +54,21 @@ hipError_t launch_face_fluxes<double>(int ndim, int kind, const flux::MeshView<d
                                       hipStream_t s) {
     if(m.F <= 0) return hipSuccess;
     const mixed::CF cf = mixed::make_cf(c);
-#define SFX_FACE(ND, K)                                                                    \
-    hipLaunchKernelGGL((flux::face_flux_kernel<ND, K, 0, double, double>), grid_for(m.F, 256), \
-                       dim3(256), 0, s, m, grad, c, cf, dQL, fstatus, ctr)
-    if(ndim == 3 && kind == 0) SFX_FACE(3, 0);
-    else if(ndim == 3) SFX_FACE(3, 1);
-    else if(kind == 0) SFX_FACE(2, 0);
-    else SFX_FACE(2, 1);
-#undef SFX_FACE
+    auto face = [&](auto nd, auto k) {
+        constexpr int ND = decltype(nd)::value, K = decltype(k)::value;
+        with_root<K == 0>(c, [&](auto root) {
+            hipLaunchKernelGGL((flux::face_flux_kernel<ND, K, 0, double, double, false,
+                                                       decltype(root)::value>),
+                               grid_for(m.F, 256), dim3(256), 0, s, m, grad, c, cf, dQL, fstatus,
+                               ctr);
+        });
+    };
+    const std::integral_constant<int, 0> exact;
+    const std::integral_constant<int, 1> hllc;
+    const std::integral_constant<int, 2> d2;
+    const std::integral_constant<int, 3> d3;
+    if(ndim == 3) kind == 0 ? face(d3, exact) : face(d3, hllc);
+    else kind == 0 ? face(d2, exact) : face(d2, hllc);
     return hipGetLastError();
 }
 

@@ -1368,13 +1368,14 @@ __device__ __forceinline__ void load_grad(const T* grad, int64_t C, int64_t cell
 // The activity flag read for every cell of a mesh without an activity array.
 static __device__ const uint8_t kAllActive = 1;
 
-// MIXED: 0 = FP64 parity solvers, 1 = mixed solvers (and, for a periodic
+// ROOT: Consts::root of the FP64 exact solver (fp64::ex_solve; unused by the
+// others).  MIXED: 0 = FP64 parity solvers, 1 = mixed solvers (and, for a periodic
 // face whose other copy has a lower index, no evaluation: the gather applies
 // that copy's flux with the opposite sign).
 // Face f: its flux goes to dQL[(f + qshift) * NC ...]; the gradients of its
 // cells are read at grad[(cell + gshift) * ND * NC ...]; the solver counters
 // are added to cnt.
-template <int ND, int KIND, int MIXED, typename T, typename R, bool FREC = false>
+template <int ND, int KIND, int MIXED, typename T, typename R, bool FREC = false, int ROOT = 0>
 __device__ __forceinline__ void face_item(const MeshView<T>& m, int64_t f,
                                           const T* __restrict__ grad, int64_t gshift,
                                           const Consts& cd, const mixed::CF& cf,
@@ -1570,8 +1571,8 @@ __device__ __forceinline__ void face_item(const MeshView<T>& m, int64_t f,
                     wr[k] = (double)WR[k];
                 }
                 if(KIND == 0)
-                    st |= fp64::ex_solve_for_flux<ND>(cd, wl, wr, n64, v64, !has_r, flux, iters,
-                                                      brent, vac);
+                    st |= fp64::ex_solve_for_flux<ND, ROOT>(cd, wl, wr, n64, v64, !has_r, flux,
+                                                            iters, brent, vac);
                 else
                     st |= fp64::hllc_solve_for_flux<ND>(cd, wl, wr, n64, v64, !has_r, flux, vac);
             } else {
@@ -1669,8 +1670,17 @@ __device__ __forceinline__ void face_item(const MeshView<T>& m, int64_t f,
     cnt[CNT_NFAIL] += fail;
 }
 
-template <int ND, int KIND, int MIXED, typename T, typename R, bool FREC = false>
-__global__ __launch_bounds__(256) void face_flux_kernel(MeshView<T> m, const T* __restrict__ grad,
+// Waves per SIMD a face kernel is held to: the FP64 exact solver's
+// out-of-line general path would otherwise set the register count (244, two
+// waves; the kernel's own code needs 150 in 3D); the others as they come.
+template <int ND, int KIND, int MIXED>
+constexpr int face_waves() {
+    return KIND == 0 && MIXED == 0 ? (ND == 2 ? 4 : 3) : 1;
+}
+
+template <int ND, int KIND, int MIXED, typename T, typename R, bool FREC = false, int ROOT = 0>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(face_waves<ND, KIND, MIXED>(), 10))) void face_flux_kernel(MeshView<T> m, const T* __restrict__ grad,
                                                         Consts cd, mixed::CF cf,
                                                         T* __restrict__ dQL,
                                                         uint8_t* __restrict__ fstatus,
@@ -1678,7 +1688,7 @@ __global__ __launch_bounds__(256) void face_flux_kernel(MeshView<T> m, const T* 
     const int64_t f = xcd_block() * blockDim.x + threadIdx.x;
     unsigned cnt[CNT_N] = {0u, 0u, 0u, 0u, 0u};
     if(f < m.F)
-        face_item<ND, KIND, MIXED, T, R, FREC>(m, f, grad, 0, cd, cf, dQL, 0, fstatus, cnt);
+        face_item<ND, KIND, MIXED, T, R, FREC, ROOT>(m, f, grad, 0, cd, cf, dQL, 0, fstatus, cnt);
     block_add_counters(ctr, cnt);
 }
 

@@ -1,14 +1,15 @@
 // riemann_fp64.hip -- plain FP64 Riemann solvers for gfx950.
 //
-// Compiled with -ffp-contract=off: every expression keeps the association of
+// Compiled with -ffp-contract=off: expressions keep the association of
 // the reference (Shadowfax src/riemann/ExactRiemannSolver.cpp,
 // src/riemann/HLLCRiemannSolver.cpp), so results differ from the CPU
-// reference only where the device pow() rounds differently from glibc.
+// reference only by round-off: the exact solver runs the same iteration over
+// a cheaper pressure function (riemann_fp64_impl.h).
 //
 // One lane per problem, SoA loads/stores (fully coalesced, 144 B per 3D
 // problem with v = 0).  The exact solver's Newton/Brent loops run per lane
-// with an iteration cap; divergence handling is left to the hardware here
-// (this is the parity path; the mixed path is the fast one).
+// with an iteration cap; divergence handling is left to the hardware.
+
 #include "riemann_fp64_impl.h"
 #include "sfx_device.h"
 #include "sfx_launch.h"
@@ -18,8 +19,9 @@ namespace fp64 {
 
 // --------------------------------------------------------------- kernels --
 
-template <int ND, int KIND>
-__global__ __launch_bounds__(256) void solve_for_flux_kernel(
+template <int ND, int KIND, int ROOT = 0>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void
+solve_for_flux_kernel(
         Consts c, int64_t N, const double* __restrict__ WL, const double* __restrict__ WR,
         const double* __restrict__ n, const double* __restrict__ v,
         const uint8_t* __restrict__ refl, double* __restrict__ F,
@@ -43,7 +45,7 @@ __global__ __launch_bounds__(256) void solve_for_flux_kernel(
         const bool r = refl ? refl[i] != 0 : false;
         uint8_t st;
         if(KIND == 0)
-            st = ex_solve_for_flux<ND>(c, wl, wr, nn, vv, r, f, iters, brent, vac);
+            st = ex_solve_for_flux<ND, ROOT>(c, wl, wr, nn, vv, r, f, iters, brent, vac);
         else
             st = hllc_solve_for_flux<ND>(c, wl, wr, nn, vv, r, f, vac);
 #pragma unroll
@@ -55,8 +57,8 @@ __global__ __launch_bounds__(256) void solve_for_flux_kernel(
     block_add_counters(ctr, cv);
 }
 
-template <int ND>
-__global__ __launch_bounds__(256) void exact_solve_kernel(
+template <int ND, int ROOT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void exact_solve_kernel(
         Consts c, int64_t N, const double* __restrict__ WL, const double* __restrict__ WR,
         const double* __restrict__ n, const uint8_t* __restrict__ refl,
         double* __restrict__ Whalf, double* __restrict__ WRout, double* __restrict__ mach_io,
@@ -75,7 +77,7 @@ __global__ __launch_bounds__(256) void exact_solve_kernel(
 #pragma unroll
         for(int d = 0; d < ND; d++) nn[d] = n[d * N + i];
         double mach = mach_io ? mach_io[i] : 0.;
-        uint8_t st = ex_solve<ND>(c, wl, wr, nn, refl ? refl[i] != 0 : false, w, &mach,
+        uint8_t st = ex_solve<ND, ROOT>(c, wl, wr, nn, refl ? refl[i] != 0 : false, w, &mach,
                                   iters, brent, vac);
 #pragma unroll
         for(int k = 0; k < NC; k++) {
@@ -104,18 +106,19 @@ hipError_t launch_solve_for_flux_fp64(int kind, int ndim, const Consts& c, int64
     if(N <= 0) return hipSuccess;
     const int bs = 256;
     dim3 grid(nblocks(N, bs)), block(bs);
-    if(ndim == 3 && kind == 0)
-        hipLaunchKernelGGL((fp64::solve_for_flux_kernel<3, 0>), grid, block, 0, stream, c, N,
-                           WL, WR, n, v, refl, F, status, ctr);
-    else if(ndim == 3)
-        hipLaunchKernelGGL((fp64::solve_for_flux_kernel<3, 1>), grid, block, 0, stream, c, N,
-                           WL, WR, n, v, refl, F, status, ctr);
-    else if(kind == 0)
-        hipLaunchKernelGGL((fp64::solve_for_flux_kernel<2, 0>), grid, block, 0, stream, c, N,
-                           WL, WR, n, v, refl, F, status, ctr);
-    else
-        hipLaunchKernelGGL((fp64::solve_for_flux_kernel<2, 1>), grid, block, 0, stream, c, N,
-                           WL, WR, n, v, refl, F, status, ctr);
+    auto solve = [&](auto nd, auto k) {
+        constexpr int ND = decltype(nd)::value, K = decltype(k)::value;
+        with_root<K == 0>(c, [&](auto root) {
+            hipLaunchKernelGGL((fp64::solve_for_flux_kernel<ND, K, decltype(root)::value>), grid,
+                               block, 0, stream, c, N, WL, WR, n, v, refl, F, status, ctr);
+        });
+    };
+    const std::integral_constant<int, 0> exact;
+    const std::integral_constant<int, 1> hllc;
+    const std::integral_constant<int, 2> d2;
+    const std::integral_constant<int, 3> d3;
+    if(ndim == 3) kind == 0 ? solve(d3, exact) : solve(d3, hllc);
+    else kind == 0 ? solve(d2, exact) : solve(d2, hllc);
     return hipGetLastError();
 }
 
@@ -126,12 +129,15 @@ hipError_t launch_exact_solve_fp64(int ndim, const Consts& c, int64_t N, const d
     if(N <= 0) return hipSuccess;
     const int bs = 256;
     dim3 grid(nblocks(N, bs)), block(bs);
-    if(ndim == 3)
-        hipLaunchKernelGGL((fp64::exact_solve_kernel<3>), grid, block, 0, stream, c, N, WL,
-                           WR, n, refl, Whalf, WRout, mach, status, ctr);
-    else
-        hipLaunchKernelGGL((fp64::exact_solve_kernel<2>), grid, block, 0, stream, c, N, WL,
-                           WR, n, refl, Whalf, WRout, mach, status, ctr);
+    with_root<true>(c, [&](auto root) {
+        constexpr int ROOT = decltype(root)::value;
+        if(ndim == 3)
+            hipLaunchKernelGGL((fp64::exact_solve_kernel<3, ROOT>), grid, block, 0, stream, c, N,
+                               WL, WR, n, refl, Whalf, WRout, mach, status, ctr);
+        else
+            hipLaunchKernelGGL((fp64::exact_solve_kernel<2, ROOT>), grid, block, 0, stream, c, N,
+                               WL, WR, n, refl, Whalf, WRout, mach, status, ctr);
+    });
     return hipGetLastError();
 }
 

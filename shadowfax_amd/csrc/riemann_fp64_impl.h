@@ -19,6 +19,40 @@
 namespace sfx {
 namespace fp64 {
 
+// ---- FP64 quotients and roots from the hardware's estimates -----------
+//
+// v_rcp_f64 and v_rsq_f64 give about 2^-24; one step of third order takes
+// that to the rounding error of the last two operations (about 1 ulp; half
+// an ulp with the residual's correction, div_by and sqrt64), in 4 to 9
+// instructions where the IEEE divide and square root take 12 and 22.  For x > 0 away from the ends of the exponent
+// range (no scaling): only ex_solve uses them, on the states it has tested.
+
+__device__ __forceinline__ double rcp64(double x) {
+    const double r = __builtin_amdgcn_rcp(x);
+    const double e = fma(-x, r, 1.0);
+    return fma(r, fma(e, e, e), r);
+}
+// a/b from r, 1/b to about an ulp: the product and its residual's correction
+__device__ __forceinline__ double div_by(double a, double b, double r) {
+    const double q = a * r;
+    return fma(fma(-b, q, a), r, q);
+}
+__device__ __forceinline__ double div64(double a, double b) { return div_by(a, b, rcp64(b)); }
+// the correction of the estimate y of 1/sqrt(x), t = x y, in units of y
+__device__ __forceinline__ double rsq_step(double t, double y) {
+    const double e = fma(-t, y, 1.0);
+    return e * fma(0.375, e, 0.5);
+}
+__device__ __forceinline__ double rsq64(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    return fma(y, rsq_step(x * y, y), y);
+}
+__device__ __forceinline__ double sqrt64(double x) {
+    const double y = __builtin_amdgcn_rsq(x), t = x * y;
+    const double q = fma(t, rsq_step(t, y), t);
+    return fma(fma(-q, q, x), 0.5 * y, q);
+}
+
 template <int ND>
 struct S {
     static constexpr int NC = ND + 2;
@@ -265,26 +299,18 @@ __device__ uint8_t ex_solve_vacuum(const Consts& c, const double* WL, const doub
     return ex_check<ND>(sol);
 }
 
-// ExactRiemannSolver::solve, ExactRiemannSolver.cpp:108-290.
+// ExactRiemannSolver::solve, ExactRiemannSolver.cpp:108-290, step by step
+// (Newton's method, then BrentsMethodSolve): the path of the problems that
+// ex_solve's iteration does not take.
 // Counters: iters (Newton+Brent steps), brent (0/1), vac (0/1).
 template <int ND>
-__device__ uint8_t ex_solve(const Consts& c, const double* WL, double* WR, const double* n,
-                            bool reflective, double* sol, double* mach,
-                            unsigned& iters, unsigned& brent, unsigned& vac) {
+__device__ uint8_t ex_solve_steps(const Consts& c, const double* WL, const double* WR,
+                                  const double* n, double vL, double vR, double* sol,
+                                  double* mach, unsigned& iters, unsigned& brent,
+                                  unsigned& vac) {
     SFX_FP64_STRICT
     const int NC = S<ND>::NC, P = S<ND>::P;
     uint8_t st = 0;
-    double vL = WL[1] * n[0] + WL[2] * n[1];
-    double vR = WR[1] * n[0] + WR[2] * n[1];
-    if(ND == 3) {
-        vL = WL[1] * n[0] + WL[2] * n[1] + WL[3] * n[ND - 1];
-        vR = WR[1] * n[0] + WR[2] * n[1] + WR[3] * n[ND - 1];
-    }
-    if(reflective) {
-#pragma unroll
-        for(int k = 0; k < NC; k++) WR[k] = WL[k];
-        vR = -vL;
-    }
     double aL = ex_soundspeed<ND>(c, WL);
     double aR = ex_soundspeed<ND>(c, WR);
     if(!(WL[0] != 0.) || !(WR[0] != 0.)) {
@@ -410,8 +436,405 @@ __device__ uint8_t ex_solve(const Consts& c, const double* WL, double* WR, const
     return st;
 }
 
-// solve_for_flux + get_flux, ExactRiemannSolver.cpp:815-880
+// ---- the exact solver's own iteration ----------------------------------
+//
+// The reference's iteration -- guess, Newton steps, Brent's method over
+// [0, guess] from a guess right of the root -- with the same tests, so that
+// it ends at the same iterate (Brent's method stops up to 1e-8 from the
+// root: in 1 of 20,000 problems its flux is more than 1e-12 from the root's),
+// over a pressure function that costs a third.  With n = 2 gamma/(gamma-1)
+// and in units of a side's own pressure, x = p/pK,
+//   shock:        f = aK k (x - 1)/sqrt(x + (g-1)/(g+1)),  k^2 = 2/(g (g+1))
+//   rarefaction:  f = 2 aK/(g-1) (y - 1),  y = x^(1/n),  x f' = aK/g y
+// one inverse square root or one n-th root a side and step, values and
+// derivative together, where pow() was called for each (226 instructions a
+// call).  A guess whose f is round-off
+// (two rarefactions: the guess is the exact root) is taken as it is; Brent's
+// method halves its bracket down to it in 27 to 30 steps.
+//
+// What bounds the batch: VALU issue; the slowest lane of a wave sets its
+// steps (8 Newton steps and about 10 of Brent's method, in the 10% of the
+// problems that take it).  Step by step (pow, IEEE quotients) -> here:
+// 262,144 problems of log-uniform states 280 -> 48 us (their 38 MB need 7),
+// 4,194,304 with vacuum and shocks 3264 -> 480 us, 1,000 problems 157 -> 26 us;
+// 4 waves per SIMD (128 VGPRs; the general path alone would take 244).
+// Normwise error against long double, 80,000 problems: rms 1.74e-14 (gamma
+// 5/3) and 5.7e-15 (7/5), maximum 3.4e-12 and 1.0e-12 both ways -- Brent's
+// stopping error -- and median 1.0e-16 both ways.
+//
+// Problems with a zero, negative, non-finite or extreme density or pressure
+// go through ex_solve_steps, whose comparisons decide as the reference's do on
+// NaNs; so do sides whose sound speeds are 1e8 apart, where the fast side's
+// round-off decides the slow side's branches, and problems whose iterates
+// leave the range of the root's FP32 seed.
+
+// x^(1/n) for x in FP32 range and rx = 1/x to 2^-40 or better: from the FP32
+// estimate y0 (relative error below 4e-6) by the series of (1 - d)^(-1/n),
+// d = 1 - y0^n/x, whose third term is below round-off; rootk carries what the
+// rounded gamma's exponent differs from 1/n by
+template <int ROOT>
+__device__ __forceinline__ double root_n(const Consts& c, double x, double rx) {
+    if constexpr(ROOT != 0) {
+        const float lf = __builtin_amdgcn_logf((float)x);
+        const double y = (double)__builtin_amdgcn_exp2f(c.rootf * lf);
+        const double y2 = y * y;
+        const double d = fma(-(y2 * y2), ROOT == 7 ? y2 * y : y, x) * rx;
+        return fma(y, fma(d, fma(d, c.rn2, c.rn), (double)(c.rootk * lf)), y);
+    }
+    (void)rx;
+    return pow(x, c.gm1d2g);
+}
+// a b + the rounding error of a b, into lo
+__device__ __forceinline__ double mul_err(double a, double b, double& lo) {
+    const double h = a * b;
+    lo = fma(a, b, -h);
+    return h;
+}
+// b^(2/(g-1)) and b^(2g/(g-1)), b >= 0; products with their rounding errors
+// carried along (plain ones would lose the digits that pow() keeps)
+template <int ROOT>
+__device__ __forceinline__ void fan_powers(const Consts& c, double b, double& r, double& p) {
+    if constexpr(ROOT != 0) {
+        double e2, e3, e5, e7;
+        const double b2 = mul_err(b, b, e2), b3 = mul_err(b2, b, e3), l3 = fma(e2, b, e3);
+        const double b5 = mul_err(b3, b2, e5), l5 = fma(l3, b2, fma(b3, e2, e5));
+        if(ROOT == 5) {
+            r = b3 + l3;
+            p = b5 + l5;
+        } else {
+            const double b7 = mul_err(b5, b2, e7);
+            r = b5 + l5;
+            p = b7 + fma(l5, b2, fma(b5, e2, e7));
+        }
+    } else {
+        r = pow(b, c.tdgm1);
+        p = pow(b, c.tgdgm1);
+    }
+}
+
+struct ExSide {
+    double p, rp, ta, ak, ag;  // pK, 1/pK, 2 aK/(g-1), k aK, aK/g
+};
+__device__ __forceinline__ ExSide ex_side(const Consts& c, double p, double rp, double a) {
+    return {p, rp, c.tdgm1 * a, c.kshock * a, c.ginv * a};
+}
+// value, p times the derivative, and y (rarefaction)
+template <int ROOT>
+__device__ __forceinline__ void ex_side_f(const Consts& c, const ExSide& s, double p, double& f,
+                                          double& pdf, double& y) {
+    const double x = div_by(p, s.p, s.rp);
+    if(p > s.p) {
+        const double r = rsq64(x + c.gm1dgp1), xm = div_by(p - s.p, s.p, s.rp), ar = s.ak * r;
+        f = xm * ar;
+        pdf = x * ar * fma(-0.5 * xm, r * r, 1.0);
+    } else {
+        double rx = __builtin_amdgcn_rcp(x);
+        rx = fma(fma(-x, rx, 1.0), rx, rx);
+        y = root_n<ROOT>(c, x, rx);
+        f = s.ta * (y - 1.0);
+        pdf = s.ag * y;
+    }
+}
+
+// the value alone
+template <int ROOT>
+__device__ __forceinline__ double ex_side_v(const Consts& c, const ExSide& s, double p) {
+    const double x = div_by(p, s.p, s.rp);
+    if(p > s.p) return div_by(p - s.p, s.p, s.rp) * (s.ak * rsq64(x + c.gm1dgp1));
+    double rx = __builtin_amdgcn_rcp(x);
+    rx = fma(fma(-x, rx, 1.0), rx, rx);
+    return s.ta * (root_n<ROOT>(c, x, rx) - 1.0);
+}
+
+// BrentsMethodSolve over [0, b], f(0) = fa < 0 < fb = f(b) (ExactRiemann-
+// Solver.cpp:462-546); the inverse quadratic interpolation over one common
+// denominator.  False: an iterate left the range of the root's seed.
+template <int ROOT>
+__device__ __forceinline__ bool ex_brent_root(const Consts& c, const ExSide& lo, const ExSide& hi,
+                                              double dv, double fa, double fb, double& b,
+                                              unsigned& iters, uint8_t& st) {
+    const double tol = c.tol;
+    double a = 0.0, d = 1e230;
+    if(fabs(fa) < fabs(fb)) {
+        a = b;
+        b = 0.0;
+        const double t = fa;
+        fa = fb;
+        fb = t;
+    }
+    double cc = a, fc = fa;
+    bool mflag = true;
+    int it = 0;
+    while(!(fb == 0) && (fabs(a - b) > tol * (a + b) * 0.5)) {
+        if(++it > c.itercap) {
+            st |= ST_ITERCAP;
+            break;
+        }
+        double s;
+        if((fa != fc) && (fb != fc)) {
+            const double ab = fa - fb, ac = fa - fc, bc = fb - fc;
+            s = (a * fb * fc * bc - b * fa * fc * ac + cc * fa * fb * ab) * rcp64(ab * ac * bc);
+        } else {
+            s = b - fb * (b - a) * rcp64(fb - fa);
+        }
+        const double tmp2 = (3. * a + b) * 0.25;
+        const double sb = fabs(s - b), bcc = mflag ? b - cc : cc - d, bsum = mflag ? b + cc : cc + d;
+        if(!(((s > tmp2) && (s < b)) || ((s < tmp2) && (s > b))) || sb >= fabs(bcc) * 0.5 ||
+           fabs(bcc) < tol * bsum * 0.5) {
+            s = (a + b) * 0.5;
+            mflag = true;
+        } else {
+            mflag = false;
+        }
+        if(!(s * hi.rp >= 1e-36)) return false;
+        const double fs = ex_side_v<ROOT>(c, lo, s) + ex_side_v<ROOT>(c, hi, s) + dv;
+        d = cc;
+        cc = b;
+        fc = fb;
+        if(fa * fs < 0.) {
+            b = s;
+            fb = fs;
+        } else {
+            a = s;
+            fa = fs;
+        }
+        if(fabs(fa) < fabs(fb)) {
+            double t = a;
+            a = b;
+            b = t;
+            t = fa;
+            fa = fb;
+            fb = t;
+        }
+    }
+    iters += it;
+    return true;
+}
+
+// where the half state lies: outside its side's wave, behind a shock, inside
+// a rarefaction fan, in the star region; or vacuum
+enum : int { EX_OUT = 0, EX_SHOCK = 1, EX_FAN = 2, EX_STAR = 3, EX_ZERO = 4 };
+
+// ex_solve_steps out of line: its registers and code are not the others'
 template <int ND>
+struct ExGeneral {
+    double WL[ND + 2], WR[ND + 2], n[ND], vL, vR, sol[ND + 2], mach;
+    unsigned iters, brent, vac;
+};
+template <int ND>
+__device__ __attribute__((noinline)) uint8_t ex_solve_general(Consts c, ExGeneral<ND>* g) {
+    return ex_solve_steps<ND>(c, g->WL, g->WR, g->n, g->vL, g->vR, g->sol, &g->mach, g->iters,
+                              g->brent, g->vac);
+}
+
+// ExactRiemannSolver::solve.  Counters: iters (Newton steps), brent (0/1: the
+// problems the reference hands to BrentsMethodSolve), vac (0/1).
+// ROOT: the solver's Consts::root (0 for any gamma), a template parameter so
+// that the 226 instructions of each pow() and their registers stay out of the
+// two gases' kernels.
+template <int ND, int ROOT>
+__device__ __forceinline__ uint8_t ex_solve(const Consts& c, const double* WL, double* WR,
+                                            const double* n, bool reflective, double* sol,
+                                            double* mach, unsigned& iters, unsigned& brent,
+                                            unsigned& vac) {
+    SFX_FP64_STRICT
+    constexpr int NC = S<ND>::NC, P = S<ND>::P;
+    double vL = WL[1] * n[0] + WL[2] * n[1];
+    double vR = WR[1] * n[0] + WR[2] * n[1];
+    if(ND == 3) {
+        vL = WL[1] * n[0] + WL[2] * n[1] + WL[3] * n[ND - 1];
+        vR = WR[1] * n[0] + WR[2] * n[1] + WR[3] * n[ND - 1];
+    }
+    if(reflective) {
+#pragma unroll
+        for(int k = 0; k < NC; k++) WR[k] = WL[k];
+        vR = -vL;
+    }
+    const double rL = WL[0], pL = WL[P], rR = WR[0], pR = WR[P];
+    // the states the iteration below is written for (false for NaNs)
+    constexpr double TINY = 1e-100, HUGE_ = 1e100;
+    const double rmax = smax(rL, rR), pmin = smin(pL, pR),
+                 pmax = smax(pL, pR);
+    bool general = !(rL >= TINY && rR >= TINY && rmax <= HUGE_ && pL >= TINY && pR >= TINY &&
+                     pmax <= HUGE_ && fabs(vL) <= HUGE_ && fabs(vR) <= HUGE_ &&
+                     pmax <= 1e24 * pmin);
+    int mode = EX_ZERO;
+    bool right = false;
+    double p = 0.0, u = 0.0, y = 0.0, aL = 0.0, aR = 0.0, rpL = 0.0, rpR = 0.0;
+    unsigned it = 0, br = 0, vc = 0;
+    uint8_t st = 0;
+    if(!general) {
+        aL = sqrt64(div64(c.gamma * pL, rL));
+        aR = sqrt64(div64(c.gamma * pR, rR));
+        rpL = rcp64(pL);
+        rpR = rcp64(pR);
+        const double dv = vR - vL;
+        general = !(smax(aL, aR) <= 1e8 * smin(aL, aR));
+        if(general) {
+        } else if(c.tdgm1 * aL + c.tdgm1 * aR <= dv) {
+            // solve_vacuum, both sides gas (ExactRiemannSolver.cpp:395-440)
+            vc = 1;
+            const double SR = vR - c.tdgm1 * aR, SL = vL + c.tdgm1 * aL;
+            right = !(SL >= 0.);
+            if(SR > 0. && SL < 0.)
+                mode = EX_ZERO;
+            else
+                mode = (right ? -aR < vR : aL > vL) ? EX_FAN : EX_OUT;
+        } else {
+            // the sides by pressure: the lower one is a shock and the higher
+            // one a rarefaction in most problems that take several steps, so
+            // a wave's lanes run the same halves of ex_side_f
+            const bool swap = pL > pR;
+            const ExSide lo = ex_side(c, pmin, swap ? rpR : rpL, swap ? aR : aL);
+            const ExSide hi = ex_side(c, pmax, swap ? rpL : rpR, swap ? aL : aR);
+            // initial guess, ExactRiemannSolver.cpp:644-673
+            const double psum = pL + pR, pfloor = c.tol * 0.5 * psum;
+            const double ppv = smax(pfloor, 0.5 * psum - 0.125 * dv * (rL + rR) * (aL + aR));
+            double pg;
+            if(pmax <= 2. * pmin && pmin <= ppv && ppv <= pmax) {
+                pg = ppv;
+            } else if(ppv < pmin) {
+                // two rarefactions, in units of the lower pressure
+                const double x = div_by(pmin, hi.p, hi.rp);
+                double rx = __builtin_amdgcn_rcp(x);
+                rx = fma(fma(-x, rx, 1.0), rx, rx);
+                const double q = root_n<ROOT>(c, x, rx);
+                const double w = div64(lo.ta + hi.ta - dv, hi.ta * q + lo.ta);
+                double wr, wp;
+                fan_powers<ROOT>(c, w, wr, wp);
+                pg = pmin * wp;
+            } else {
+                const double gl = lo.ak * __builtin_amdgcn_rsq(fma(ppv, lo.rp, c.gm1dgp1)),
+                             gh = hi.ak * __builtin_amdgcn_rsq(fma(ppv, hi.rp, c.gm1dgp1));
+                pg = (gl + gh - dv) * __builtin_amdgcn_rcp(gl * lo.rp + gh * hi.rp);
+            }
+            pg = smax(pfloor, pg);
+            double flo, fhi, dlo, dhi, ylo = 1.0, yhi = 1.0;
+            const double f0 = -lo.ta - hi.ta + dv;
+            const bool pure = f0 < c.cutoff;
+            for(;;) {
+                // outside the seed's range, or not a number
+                if(!(pg * hi.rp >= 1e-36 && pg * lo.rp <= 1e36)) {
+                    general = true;
+                    break;
+                }
+                ex_side_f<ROOT>(c, lo, pg, flo, dlo, ylo);
+                ex_side_f<ROOT>(c, hi, pg, fhi, dhi, yhi);
+                const double f = flo + fhi + dv;
+                if(!(fabs(p - pg) > c.tol * 0.5 * (p + pg)) || f == 0.0) break;
+                if(f > 0.0 && !pure) {
+                    br = 1;
+                    if(f <= 5e-16 * (lo.ta + hi.ta + fabs(flo) + fabs(fhi))) break;
+                    p = pg;
+                    if(!ex_brent_root<ROOT>(c, lo, hi, dv, f0, f, pg, it, st)) {
+                        general = true;
+                        break;
+                    }
+                    // once more round the loop, for the sides' values there
+                    p = pg;
+                    continue;
+                }
+                if(++it > (unsigned)c.itercap) {
+                    st |= ST_ITERCAP;
+                    break;
+                }
+                p = pg;
+                // (a step quotient off by 2^-24 lands right of the root)
+                pg = fma(-p, f * rcp64(dlo + dhi), p);
+                if(pg < 0.0) {
+                    // clamped to 0, where f' is infinite: the pure Newton
+                    // iteration ends there (ExactRiemannSolver.cpp:146-154)
+                    pg = 0.0;
+                    flo = -lo.ta;
+                    fhi = -hi.ta;
+                    ylo = yhi = 0.0;
+                    break;
+                }
+            }
+            p = pg;
+            const double fl = swap ? fhi : flo, fr = swap ? flo : fhi;
+            u = 0.5 * (vL + vR) + 0.5 * (fr - fl);
+            right = u < 0.;
+            y = (right != swap) ? yhi : ylo;
+        }
+    }
+    if(general) {
+        ExGeneral<ND> g;
+#pragma unroll
+        for(int k = 0; k < NC; k++) {
+            g.WL[k] = WL[k];
+            g.WR[k] = WR[k];
+        }
+#pragma unroll
+        for(int d = 0; d < ND; d++) g.n[d] = n[d];
+        g.vL = vL;
+        g.vR = vR;
+        g.mach = mach ? *mach : 0.0;
+        g.iters = iters;
+        g.brent = brent;
+        g.vac = vac;
+        st = ex_solve_general<ND>(c, &g);
+#pragma unroll
+        for(int k = 0; k < NC; k++) sol[k] = g.sol[k];
+        if(mach) *mach = g.mach;
+        iters = g.iters;
+        brent = g.brent;
+        vac = g.vac;
+        return st;
+    }
+    iters += it;
+    brent |= br;
+    vac |= vc;
+    // sampling at x/t = 0, ExactRiemannSolver.cpp:190-271
+    const double sgn = right ? 1.0 : -1.0, aK = right ? aR : aL, uK = right ? vR : vL;
+#pragma unroll
+    for(int k = 0; k < NC; k++) sol[k] = right ? WR[k] : WL[k];
+    const double rK = sol[0], pK = sol[P], x = div_by(p, pK, right ? rpR : rpL);
+    double vhalf = 0.0;
+    if(!vc) {
+        if(mach) {
+            if(p > pL) *mach = smax(*mach, sqrt(c.gp1d2g * p / pL + c.gm1d2g));
+            if(p > pR) *mach = smax(*mach, sqrt(c.gp1d2g * p / pR + c.gm1d2g));
+        }
+        mode = EX_OUT;
+        if(p > pK) {
+            if(fma(sgn, uK, aK * sqrt64(fma(c.gp1d2g, x, c.gm1d2g))) > 0.) mode = EX_SHOCK;
+        } else if(fma(sgn, uK, aK) > 0.) {
+            const double ST = fma(sgn * aK, y, u);
+            mode = (right ? ST <= 0. : ST > 0.) ? EX_FAN : EX_STAR;
+        }
+    }
+    if(mode == EX_FAN) {
+        const double base = c.tdgp1 - div64(sgn * c.gm1dgp1 * uK, aK);
+        double br_, bp;
+        fan_powers<ROOT>(c, base, br_, bp);
+        sol[0] = rK * br_;
+        sol[P] = pK * bp;
+        vhalf = c.tdgp1 * (-sgn * aK + c.gm1d2 * uK) - uK;
+    } else if(mode == EX_SHOCK || mode == EX_STAR) {
+        if(mode == EX_SHOCK) {
+            sol[0] = div64(rK * (x + c.gm1dgp1), fma(c.gm1dgp1, x, 1.0));
+        } else {
+            // x^(1/g) = x/y^2 = y^(n-2) (n = 7: y^5 would carry 5 times y's error)
+            const double y2 = y * y;
+            sol[0] = ROOT == 5   ? rK * (y2 * y)
+                     : ROOT == 7 ? (y > 0. ? div64(rK * x, y2) : 0.)
+                                 : rK * pow(x, c.ginv);
+        }
+        sol[P] = p;
+        vhalf = u - uK;
+    } else if(mode == EX_ZERO) {
+#pragma unroll
+        for(int k = 0; k < NC; k++) sol[k] = 0.;
+    }
+#pragma unroll
+    for(int d = 0; d < ND; d++) sol[1 + d] += vhalf * n[d];
+    st |= ex_check<ND>(sol);
+    return st;
+}
+
+// solve_for_flux + get_flux, ExactRiemannSolver.cpp:815-880
+template <int ND, int ROOT>
 __device__ uint8_t ex_solve_for_flux(const Consts& c, const double* WL, double* WR,
                                      const double* n, const double* v, bool reflective,
                                      double* F, unsigned& iters, unsigned& brent,
@@ -420,7 +843,7 @@ __device__ uint8_t ex_solve_for_flux(const Consts& c, const double* WL, double* 
     const int NC = S<ND>::NC, P = S<ND>::P;
     double W[NC];
     double maxmach = 0.;
-    uint8_t st = ex_solve<ND>(c, WL, WR, n, reflective, W, &maxmach, iters, brent, vac);
+    uint8_t st = ex_solve<ND, ROOT>(c, WL, WR, n, reflective, W, &maxmach, iters, brent, vac);
 #pragma unroll
     for(int d = 0; d < ND; d++) W[1 + d] += v[d];
     double Fi[ND][NC];

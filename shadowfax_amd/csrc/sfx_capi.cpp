@@ -114,6 +114,14 @@ int sfx_solver_create(int kind, int ndim, double gamma, double tolerance, double
     c.itercap = 1000;
     // integer-power shortcuts of the mixed path hold when (g-1)/(2g) = 1/5
     c.fast53 = std::fabs(gamma - 5.0 / 3.0) < 1e-12;
+    for(int n : {5, 7})
+        if(std::fabs(c.tgdgm1 - n) < 1e-12 * n) c.root = n;
+    c.rn = c.root ? 1.0 / c.root : 0.0;
+    c.rn2 = 0.5 * c.rn * (1.0 + c.rn);
+    c.rootf = (float)c.rn;
+    const long double gl = gamma;
+    c.rootk = c.root ? (float)(((gl - 1) / (2 * gl) - 1.0L / c.root) * std::log(2.0L)) : 0.f;
+    c.kshock = std::sqrt(c.tdgp1 / gamma);
     hipError_t e = hipGetDevice(&h->device);
     if(e != hipSuccess) {
         delete h;

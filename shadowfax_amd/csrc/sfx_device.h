@@ -8,6 +8,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace sfx {
 
 // Solver constants derived from gamma exactly as the reference derives them
@@ -18,7 +20,24 @@ struct Consts {
     double tol, cutoff;
     int itercap;   // bound on Newton and on Brent iterations (reference: none)
     int fast53;    // gamma == 5/3: exponents 0.2, 0.6, 0.8, 3, 5 (mixed path)
+    // FP64 exact solver: 2 gamma/(gamma-1) where that is 5 (gamma = 5/3) or 7
+    // (gamma = 7/5), else 0; 1/root and (1 + 1/root)/(2 root), its root
+    // series; sqrt(2/(gamma (gamma+1)))
+    int root;
+    float rootf, rootk;  // 1/root; ((g-1)/(2g) - 1/root) ln 2
+    double rn, rn2, kshock;
 };
+
+// f(std::integral_constant<int, ROOT>) for the kernels that take Consts::root
+// as a template parameter: the FP64 exact solver's (exact), 0 for all others
+template <bool exact, class Fn>
+inline void with_root(const Consts& c, Fn f) {
+    if constexpr(exact) {
+        if(c.root == 5) return f(std::integral_constant<int, 5>());
+        if(c.root == 7) return f(std::integral_constant<int, 7>());
+    }
+    f(std::integral_constant<int, 0>());
+}
 
 // status bits, one byte per problem / face / cell
 enum : uint8_t {
