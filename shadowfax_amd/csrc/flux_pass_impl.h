@@ -68,14 +68,8 @@
 #ifndef SFX_GATHER_KB
 #define SFX_GATHER_KB 8
 #endif
-#ifndef SFX_GATHER_WAVES  // gathers of FP32 rows over large meshes: waves per SIMD (0: all that fit)
-#define SFX_GATHER_WAVES 2
-#endif
-#ifndef SFX_GATHER_WAVES_F64  // the same for FP64 rows
-#define SFX_GATHER_WAVES_F64 1
-#endif
-#ifndef SFX_GATHER_BIG  // ... of at least this many cells
-#define SFX_GATHER_BIG (1 << 20)
+#ifndef SFX_BIG_MESH  // cells from which record builds run at bounded occupancy
+#define SFX_BIG_MESH (1 << 20)
 #endif
 #ifndef SFX_EGEO_U  // entries a lane of the FP32 record build forms at a time
 #define SFX_EGEO_U 4  // (3D Sedov build: 1.49 ms; 2: 1.51, 8: 1.55, one at a time: 1.69)
@@ -88,13 +82,6 @@
 #endif
 #ifndef SFX_GATHER_KB_F64  // FP64 rows: the same registers as 8 FP32 rows
 #define SFX_GATHER_KB_F64 4
-#endif
-#ifndef SFX_GATHER_KB_BIG  // FP32 rows in flight per lane at the large meshes' bounded occupancy
-#define SFX_GATHER_KB_BIG 16  // (3D Sedov gather 251 -> 218 us; 8: 221, 32: 455, spilling;
-                              // at 1 wave per SIMD, 32: 318 us, 24: 380)
-#endif
-#ifndef SFX_GATHER_KB_BIG_F64  // the same for FP64 rows
-#define SFX_GATHER_KB_BIG_F64 8  // (409 -> 374 us; 16: 389)
 #endif
 
 namespace sfx {
@@ -1696,7 +1683,7 @@ __attribute__((amdgpu_waves_per_eu(face_waves<ND, KIND, MIXED>(), 10))) void fac
 
 // Cell i: dQ[i] = its entries' dQL[(f + qshift)] in ascending face order,
 // summed in FP64 (T: storage of dQL).
-template <int ND, int MIXED, typename T, int KB0 = 0>
+template <int ND, int MIXED, typename T>
 __device__ __forceinline__ void gather_cell(int64_t i, const int64_t* __restrict__ goff,
                                             const int32_t* __restrict__ gent,
                                             const uint8_t* __restrict__ ghost,
@@ -1712,11 +1699,11 @@ __device__ __forceinline__ void gather_cell(int64_t i, const int64_t* __restrict
 #pragma unroll
     for(int k = 0; k < NC; k++) acc[k] = 0.0;
     const int64_t j0 = goff[i], j1 = goff[i + 1];
-    // KB entries at a time (KB0, or SFX_GATHER_KB / _F64): their indices,
+    // KB entries at a time: their indices,
     // then their rows, are loaded before any is added, so a lane has that
     // many independent loads in flight; the additions keep ascending face
     // order
-    constexpr int KB = KB0 > 0 ? KB0 : (sizeof(T) == 8 ? SFX_GATHER_KB_F64 : SFX_GATHER_KB);
+    constexpr int KB = sizeof(T) == 8 ? SFX_GATHER_KB_F64 : SFX_GATHER_KB;
     for(int64_t jb = j0; jb < j1; jb += KB) {
         int32_t f[KB];
         bool neg[KB];
@@ -1770,34 +1757,107 @@ inline unsigned occupancy_lds_bytes(int waves, int64_t items, int64_t big, unsig
     const unsigned per = ((163840u / (unsigned)waves) & ~1023u) - 1024u;
     return per > static_lds ? per - static_lds : 0u;
 }
-template <typename T>
-inline unsigned gather_lds_bytes(int64_t C) {
-    return occupancy_lds_bytes(sizeof(T) == 8 ? SFX_GATHER_WAVES_F64 : SFX_GATHER_WAVES, C,
-                               SFX_GATHER_BIG, 0);
+template <int N, typename T>
+struct alignas(sizeof(T)) PackedRow {
+    T v[N];
+};
+
+// CELLS consecutive cells a block, a thread per cell and KPT components.  The
+// block's NT threads first walk the cells' entries, which lie one after
+// another in gent, U each at a time, and put each entry's row, negated where
+// the cell is the face's right one, into LDS; then every thread adds up its
+// cell's components in entry order (ascending face order, in FP64).  A block
+// with more than ROWS entries goes round again.
+//
+// The address unit takes about a cycle per lane that reads a line of its own.
+// With a lane per cell and its entries in turn, every index and row was such
+// a read (4, 16 and 4 bytes an entry, FP32 in 3D; unit busy 0.88); here the
+// indices are read 64 at a time and so are the rows of the faces that a cell
+// created, which follow one another, and dQ is written in full lines.
+// 3D Poisson mesh, 1,100,000 cells: FP32 rows 118 -> 76 us, 250,000 cells,
+// FP64 rows 52 -> 25 us; 2D, 262,144 cells, FP32 6.9 -> 5.8 us, 150,001
+// cells, FP64 8.5 -> 5.6 us.
+template <int ND, typename T, int CELLS, int NT, int KPT, int ROWS, int U>
+__global__ __launch_bounds__(NT) void gather_kernel(int64_t C, const int64_t* __restrict__ goff,
+                                                    const int32_t* __restrict__ gent,
+                                                    const T* __restrict__ dQL,
+                                                    double* __restrict__ dQ) {
+    constexpr int NC = ND + 2, TPC = NC / KPT;
+    static_assert(TPC * KPT == NC && CELLS * TPC <= NT && CELLS < NT, "threads per cell");
+    __shared__ T rows[ROWS * NC];
+    __shared__ int s_off[CELLS + 1];
+    const int64_t i0 = xcd_block() * CELLS;
+    const int nc = (int)((C - i0) < CELLS ? (C - i0) : CELLS);
+    const int t = threadIdx.x;
+    const int64_t base = goff[i0];
+    if(t <= nc) s_off[t] = (int)(goff[i0 + t] - base);
+    __syncthreads();
+    const int n = s_off[nc], c = t / TPC, k = (t - c * TPC) * KPT;
+    const bool mine = c < nc;
+    int j = mine ? s_off[c] : 0;
+    const int j1 = mine ? s_off[c + 1] : 0;
+    double acc[KPT];
+#pragma unroll
+    for(int l = 0; l < KPT; l++) acc[l] = 0.0;
+    const PackedRow<NC, T>* src = reinterpret_cast<const PackedRow<NC, T>*>(dQL);
+    for(int r0 = 0; r0 < n; r0 += ROWS) {
+        const int m = n - r0 < ROWS ? n - r0 : ROWS;
+        if(r0) __syncthreads();  // the last rows have been read
+        for(int b = t; b < m; b += U * NT) {
+            // U entries' indices, then their rows, before any is stored (past
+            // the last: that one's again)
+            int32_t e[U];
+#pragma unroll
+            for(int u = 0; u < U; u++) {
+                const int q = b + u * NT;
+                e[u] = gent[base + r0 + (q < m ? q : m - 1)];
+            }
+            PackedRow<NC, T> x[U];
+#pragma unroll
+            for(int u = 0; u < U; u++) x[u] = src[ent_face(e[u])];
+            // (sunk to its store, a row's load would wait for the one before)
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for(int u = 0; u < U; u++) {
+                const int q = b + u * NT;
+                if(q < m) {
+#pragma unroll
+                    for(int l = 0; l < NC; l++)
+                        rows[q * NC + l] = ent_right(e[u]) ? -x[u].v[l] : x[u].v[l];
+                }
+            }
+        }
+        __syncthreads();
+        const int end = j1 < r0 + m ? j1 : r0 + m;
+        for(; j < end; j++)
+#pragma unroll
+            for(int l = 0; l < KPT; l++) acc[l] += (double)rows[(j - r0) * NC + k + l];
+    }
+    if(mine) {
+#pragma unroll
+        for(int l = 0; l < KPT; l++) dQ[(i0 + c) * NC + k + l] = acc[l];
+    }
 }
 
-// waves per SIMD a gather kernel is compiled for: KB0 > 0 is the variant for
-// large meshes, which run at the bounded occupancy of gather_lds_bytes, so
-// the compiler may spend that occupancy's registers on rows in flight
-template <typename T, int KB0>
-constexpr int gather_waves() {
-    return KB0 > 0 ? (sizeof(T) == 8 ? SFX_GATHER_WAVES_F64 : SFX_GATHER_WAVES) : 0;
-}
-
-template <int ND, int MIXED, typename T, int KB0 = 0>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
-        gather_waves<T, KB0>() > 0 ? gather_waves<T, KB0>() : 1,
-        gather_waves<T, KB0>() > 0 ? gather_waves<T, KB0>() : 10))) void
-gather_kernel(int64_t C, int64_t F,
-                                                     const int64_t* __restrict__ goff,
-                                                     const int32_t* __restrict__ gent,
-                                                     const uint8_t* __restrict__ ghost,
-                                                     const int32_t* __restrict__ twin,
-                                                     const T* __restrict__ dQL,
-                                                     double* __restrict__ dQ) {
-    (void)F;
-    const int64_t i = xcd_block() * blockDim.x + threadIdx.x;
-    if(i < C) gather_cell<ND, MIXED, T, KB0>(i, goff, gent, ghost, twin, dQL, 0, dQ);
+// The block shape by dimension and row size, each the best of those measured
+// (3D FP32, 250,000 cells: 48 cells on 256 threads 16.0 us, 64 on 320 17.2,
+// 32 on 192 16.9; FP64, whose rows take twice the LDS: 32 on 192 25.1 us, 48
+// on 256 26.5, 64 on 320 37.6.  2D FP32, 150,001 cells: two components a
+// thread, 64 cells on 128 threads 4.9 us, one a thread 5.6, 128 cells 5.3).
+// ROWS holds the entries that so many cells of a Poisson mesh have (15.5 and
+// 6 each) with some to spare, U takes them in one round.
+template <int ND_, int CELLS_, int NT_, int KPT_, int ROWS_, int U_>
+struct GatherShape {
+    static constexpr int ND = ND_, CELLS = CELLS_, NT = NT_, KPT = KPT_, ROWS = ROWS_, U = U_;
+};
+template <typename T, class Fn>
+inline void gather_shape(int ndim, Fn f) {
+    if(ndim == 2)
+        f(GatherShape<2, 64, 128, 2, 448, 4>());
+    else if constexpr(sizeof(T) == 4)
+        f(GatherShape<3, 48, 256, 1, 832, 4>());
+    else
+        f(GatherShape<3, 32, 192, 1, 576, 3>());
 }
 
 // ------------------------------------------------------------ K5 update --

@@ -26,7 +26,7 @@ hipError_t launch_entry_geometry<float>(int ndim, const flux::MeshView<float>& m
         // grouped layout: a block per group of 64 cells (the last one padded)
         if(m.C <= 0) return hipSuccess;
         const dim3 g((unsigned)((m.C + 63) / 64));  // one block per group
-        const unsigned egeo_lds = flux::occupancy_lds_bytes(SFX_EGEO_WAVES, m.C, SFX_GATHER_BIG, 1024);
+        const unsigned egeo_lds = flux::occupancy_lds_bytes(SFX_EGEO_WAVES, m.C, SFX_BIG_MESH, 1024);
         if(ndim == 3)
             hipLaunchKernelGGL((flux::entry_geometry_grouped_kernel<3, float>), g, dim3(256), egeo_lds,
                                s, m, egeo);
@@ -110,22 +110,12 @@ hipError_t launch_gather_mixed(int ndim, int64_t C, int64_t F, const int64_t* go
                                const int32_t* gent, const uint8_t* ghost, const int32_t* twin,
                                const float* dQL, double* dQ, hipStream_t s) {
     if(C <= 0) return hipSuccess;
-    const unsigned lds = flux::gather_lds_bytes<float>(C);
-    // large meshes (lds > 0): the variant with more rows in flight
-    if(ndim == 3)
-        if(lds)
-            hipLaunchKernelGGL((flux::gather_kernel<3, 1, float, SFX_GATHER_KB_BIG>), grid_for(C, 256), dim3(256), lds,
-                               s, C, F, goff, gent, ghost, twin, dQL, dQ);
-        else
-            hipLaunchKernelGGL((flux::gather_kernel<3, 1, float>), grid_for(C, 256), dim3(256), lds, s,
-                           C, F, goff, gent, ghost, twin, dQL, dQ);
-    else
-        if(lds)
-            hipLaunchKernelGGL((flux::gather_kernel<2, 1, float, SFX_GATHER_KB_BIG>), grid_for(C, 256), dim3(256), lds,
-                               s, C, F, goff, gent, ghost, twin, dQL, dQ);
-        else
-            hipLaunchKernelGGL((flux::gather_kernel<2, 1, float>), grid_for(C, 256), dim3(256), lds, s,
-                           C, F, goff, gent, ghost, twin, dQL, dQ);
+    flux::gather_shape<float>(ndim, [&](auto shape) {
+        using S = decltype(shape);
+        hipLaunchKernelGGL((flux::gather_kernel<S::ND, float, S::CELLS, S::NT, S::KPT, S::ROWS, S::U>),
+                           dim3((unsigned)((C + S::CELLS - 1) / S::CELLS)), dim3(S::NT), 0, s, C, goff,
+                           gent, dQL, dQ);
+    });
     return hipGetLastError();
 }
 
