@@ -85,9 +85,43 @@ __global__ void timestep_init_kernel(uint64_t* result, uint64_t smax) {
     }
 }
 
-// One lane per cell: TimeLine::calculate_timestep's gas loop
-// (src/TimeLine.cpp:248-320).  The smallest step and the active count go to
-// result through one atomic per block.
+// The reference's step search, `S2 = M; while(interval(S2) > S) S2 >>= 1`,
+// started near its end: the interval falls with every halving, so where
+// interval(M >> k) > S still holds at the k that the exponents of tottime and
+// S give (less 2), it held at every earlier one.  0 when no step is left.
+__device__ __forceinline__ uint64_t tl_largest_step(const TimelineArgs& tl, double S) {
+    uint64_t s2 = tl.integer_maxtime;
+    const int k = __builtin_amdgcn_frexp_exp(tl.tottime) - __builtin_amdgcn_frexp_exp(S) - 2;
+    if(k > 0 && k < 64) {
+        const uint64_t near = s2 >> k;
+        if(tl_interval(tl, near) > S) s2 = near;
+    }
+    while(s2 && tl_interval(tl, s2) > S) s2 >>= 1;  // at most 64 halvings
+    return s2;
+}
+// `while(left % S2) S2 >>= 1`: the largest halving of S2 that divides what is
+// left of the time line.  For a power of two that is left's lowest set bit.
+__device__ __forceinline__ uint64_t tl_synchronise(uint64_t left, uint64_t s2) {
+    if((s2 & (s2 - 1)) == 0) {
+        const uint64_t low = left & (0 - left);
+        return (low != 0 && low < s2) ? low : s2;
+    }
+    while(left % s2) s2 >>= 1;  // S2 = 1 divides everything: at most 64 halvings
+    return s2;
+}
+
+// kTsCells cells a thread, 256 apart: one atomic a block and result then
+// stands for 1,024 cells (blocks of 256 cells put 8,192 atomics a result on
+// one address for 2,097,152 cells).
+constexpr int kTsCells = 4;
+
+// TimeLine::calculate_timestep's gas loop (src/TimeLine.cpp:248-320).  The
+// smallest step and the active count go to result through one atomic each per
+// block.  Bound by the cells' bytes (106 in 3D) and, for the cells whose step
+// starts now, cbrt and two square roots; 2,097,152 3D cells with individual
+// steps took 198 us when each active lane halved its way down from the whole
+// time line (a division a halving, a 64-bit remainder after) and take
+// 67 us (43 at copy rate).
 template <int ND, int KIND>
 __global__ __launch_bounds__(256) void timestep_kernel(
         TimelineArgs tl, double gamma, int64_t C, const double* __restrict__ W,
@@ -95,20 +129,29 @@ __global__ __launch_bounds__(256) void timestep_kernel(
         uint64_t* __restrict__ starttime, uint64_t* __restrict__ endtime, double* __restrict__ dt,
         uint8_t* __restrict__ active, uint64_t* __restrict__ result, uint8_t* __restrict__ status) {
     constexpr int NC = ND + 2, P = ND + 1;
-    __shared__ uint64_t s_min[256];
-    __shared__ unsigned s_cnt;
-    if(threadIdx.x == 0) s_cnt = 0;
-    __syncthreads();
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ uint64_t s_min[4];
+    __shared__ unsigned s_cnt[4];
     const uint64_t Smax = tl.max_timestep;
     uint64_t mine = Smax;
-    if(i < C) {
+    unsigned count = 0;
+    const int64_t i0 = (int64_t)blockIdx.x * (256 * kTsCells) + threadIdx.x;
+    uint64_t ends[kTsCells];
+#pragma unroll
+    for(int u = 0; u < kTsCells; u++) {
+        const int64_t i = i0 + u * 256;
+        ends[u] = i < C ? endtime[i] : 0;
+    }
+#pragma unroll
+    for(int u = 0; u < kTsCells; u++) {
+        const int64_t i = i0 + u * 256;
+        if(i >= C) break;
         uint8_t st = 0;
-        const uint64_t end0 = endtime[i];
+        const uint64_t end0 = ends[u];
+        uint64_t start1 = 0, end1 = end0;
         const bool act = end0 == tl.current_time + tl.timestep;
         active[i] = act ? 1 : 0;
         if(act) {
-            atomicAdd(&s_cnt, 1u);
+            count++;
             const double* w = W + i * NC;
             // v = W.v - particle velocity; Vec::norm (src/Vec.hpp:140,378)
             const double vx = w[1] - vel[i * ND], vy = w[2] - vel[i * ND + 1];
@@ -130,38 +173,50 @@ __global__ __launch_bounds__(256) void timestep_kernel(
             if(tl_interval(tl, Smax) < S) {
                 S2 = Smax;
             } else {
-                S2 = tl.integer_maxtime;
-                while(tl_interval(tl, S2) > S) S2 >>= 1;  // at most 64 halvings
+                S2 = tl_largest_step(tl, S);
                 if(!S2) {
                     st = SFX_ST_TIMESTEP;
                 } else {
-                    // S2 = 1 divides everything: at most 64 halvings
-                    while((tl.integer_maxtime - end0) % S2) S2 >>= 1;
+                    S2 = tl_synchronise(tl.integer_maxtime - end0, S2);
                     S2 = (S2 < tl.min_timestep) ? tl.min_timestep : S2;
                     S2 = (S2 > tl.max_timestep) ? tl.max_timestep : S2;
                 }
             }
             if(!st) {
-                mine = S2;
+                mine = S2 < mine ? S2 : mine;
+                start1 = end0;
+                end1 = end0 + S2;
                 if(!tl.global_timestep) {
-                    starttime[i] = end0;
-                    endtime[i] = end0 + S2;
+                    starttime[i] = start1;
+                    endtime[i] = end1;
                 }
             }
         }
         if(status) status[i] = st;
-        if(!tl.global_timestep) dt[i] = tl_realtime(tl, endtime[i] - starttime[i]);
+        if(!tl.global_timestep) {
+            if(!act || st) start1 = starttime[i];
+            dt[i] = tl_realtime(tl, end1 - start1);
+        }
     }
-    s_min[threadIdx.x] = mine;
+#pragma unroll
+    for(int off = 32; off > 0; off >>= 1) {
+        const uint64_t o = __shfl_xor(mine, off, 64);
+        mine = o < mine ? o : mine;
+        count += __shfl_xor(count, off, 64);
+    }
+    if((threadIdx.x & 63) == 0) {
+        s_min[threadIdx.x >> 6] = mine;
+        s_cnt[threadIdx.x >> 6] = count;
+    }
     __syncthreads();
-    for(int k = 128; k > 0; k >>= 1) {
-        if((int)threadIdx.x < k && s_min[threadIdx.x + k] < s_min[threadIdx.x])
-            s_min[threadIdx.x] = s_min[threadIdx.x + k];
-        __syncthreads();
-    }
     if(threadIdx.x == 0) {
-        if(s_min[0] < Smax) atomicMin((unsigned long long*)result, (unsigned long long)s_min[0]);
-        if(s_cnt) atomicAdd((unsigned long long*)(result + 1), (unsigned long long)s_cnt);
+#pragma unroll
+        for(int q = 1; q < 4; q++) {
+            mine = s_min[q] < mine ? s_min[q] : mine;
+            count += s_cnt[q];
+        }
+        if(mine < Smax) atomicMin((unsigned long long*)result, (unsigned long long)mine);
+        if(count) atomicAdd((unsigned long long*)(result + 1), (unsigned long long)count);
     }
 }
 
@@ -188,7 +243,9 @@ hipError_t launch_hydro_timestep(int kind, int ndim, double gamma, int64_t C,
     hipLaunchKernelGGL(timestep_init_kernel, dim3(1), dim3(64), 0, s, result, tl.max_timestep);
     if(C > 0) {
 #define SFX_TS(ND, K)                                                                       \
-    hipLaunchKernelGGL((timestep_kernel<ND, K>), blocks(C), dim3(256), 0, s, tl, gamma, C, W, \
+    hipLaunchKernelGGL((timestep_kernel<ND, K>),                                              \
+                       dim3((unsigned)((C + 256 * kTsCells - 1) / (256 * kTsCells))), dim3(256), 0, \
+                       s, tl, gamma, C, W,                                                  \
                        vel, volume, starttime, endtime, dt, active, result, status)
         if(ndim == 3) {
             if(kind == 1)
