@@ -382,10 +382,13 @@ typedef struct {
  * tessellation from the face arrays and cf_entry, in each cell's walk order
  * so that the pass streams them; for entry j of cell i (face f seen from
  * side s):
- *   FP64:  [area, mc (ndim), rRL seen from i (ndim), dL or dR (ndim),
- *           the neighbour's index bits (-1: mirror), (3D) pad]
+ *   FP64:  3D [dL or dR (3), area, mc (3), rRL seen from i (3), the
+ *           neighbour's index bits, pad], 2D [dL or dR (2), area, the
+ *           neighbour's index bits, mc (2), rRL seen from i (2)]
  *          -- the values the gradient loop of VorCell::estimate_gradient
- *          reads per face (src/VorCell.cpp:471-500);
+ *          reads per face (src/VorCell.cpp:471-500), d = 0 where the area
+ *          is 0; the index in the low 32 bits (-1: mirror), bit 32 set where
+ *          a component's exponent is out of +-200;
  *   mixed: [area (mc - r/2)/|r| (ndim), the neighbour's index bits
  *          (~f: mirror), (2D) pad | dL or dR (ndim), area, (2D) pad],
  *          r = rRL seen from i -- the weights of the difference form of

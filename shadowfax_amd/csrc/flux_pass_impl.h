@@ -135,7 +135,10 @@ struct MeshView {
 
 // Per-entry record of a cell's face, in the cell's walk order.  FP64
 // storage (the parity pass):
-//   [A, c (ND), r_ij (ND), d (ND), neighbour index bits, (3D: pad)]
+//   3D: [d (3), A, c (3), r_ij (3), neighbour index bits, pad]
+//   2D: [d (2), A, neighbour index bits, c (2), r_ij (2)]
+// (d = 0 where A = 0, so that the limiter reads nothing else; bit 32 of the
+// neighbour's word: c or r_ij out of the range of quot_by)
 // with c = mc, r_ij = rRL seen from the cell (-rRL for the left cell),
 // d = dL or dR, neighbour = the other cell or -1 (mirror).  FP32 storage
 // (the mixed pass, which sums the difference form of the gradient), two
@@ -154,6 +157,37 @@ template <int ND>
 struct Rec32 {
     static constexpr int G = 0, NB = ND, D = 4, A = 4 + ND, A2 = (ND == 2) ? 3 : A;
 };
+
+// the same of the FP64 record
+template <int ND>
+struct Rec64 {
+    static constexpr int D = 0, A = ND, C = (ND == 3) ? 4 : 4, R = C + ND, NB = (ND == 3) ? 10 : 3;
+};
+
+// Quotients by one divisor, bit for bit the IEEE ones: the compiler's divide
+// is an estimate of 1/b, two Newton steps, the product and its residual's
+// correction, wrapped in a scaling of operands near the ends of the exponent
+// range and a fix-up of zeros, infinities and NaNs (12 instructions).  For
+// operands that are zero or within 2^-200 .. 2^200 neither wrapper changes
+// anything, and quotients by the same b share its reciprocal: 3 instructions
+// each (a zero quotient may lose a minus sign).
+struct Recip {
+    double b, r;
+};
+__device__ __forceinline__ Recip recip_of(double b) {
+    double r = __builtin_amdgcn_rcp(b);
+    r = fma(fma(-b, r, 1.0), r, r);
+    return {b, fma(fma(-b, r, 1.0), r, r)};
+}
+__device__ __forceinline__ double quot_by(double a, const Recip& d) {
+    const double q = a * d.r;
+    return fma(fma(-d.b, q, a), d.r, q);
+}
+// x is neither zero (or below 2^-1042) nor within 2^-200 .. 2^200
+__device__ __forceinline__ bool quot_wide(double x) {
+    const uint32_t u = (uint32_t)(__double_as_longlong(x) >> 32) & 0x7fffffffu;
+    return u > ((1023u + 200u) << 20) || u - 1u < ((1023u - 200u) << 20);
+}
 
 // Row o of an item-major FP64 array of NC = 4 or 5 values per item
 // ([n][NC], 16-byte aligned base) with 16-byte loads.  For NC = 5 the row
@@ -613,17 +647,23 @@ __device__ __forceinline__ EntryVals64<ND> load_entry_vals64(const MeshView<doub
 template <int ND>
 __device__ __forceinline__ void entry_record_from_vals64(const EntryVals64<ND>& v, int32_t e,
                                                          double* rec) {
-    constexpr int ER = entry_rec(ND, false);
+    using RL = Rec64<ND>;
     const bool isR = ent_right(e);
-    rec[0] = v.area;
+    bool wide = false;
 #pragma unroll
     for(int l = 0; l < ND; l++) {
-        rec[1 + l] = v.mc[l];
-        rec[1 + ND + l] = isR ? v.rRL[l] : -v.rRL[l];
-        rec[1 + 2 * ND + l] = v.d[l];
+        rec[RL::D + l] = v.area != 0.0 ? v.d[l] : 0.0;
+        rec[RL::C + l] = v.mc[l];
+        rec[RL::R + l] = isR ? v.rRL[l] : -v.rRL[l];
+        wide |= quot_wide(v.mc[l]) | quot_wide(v.rRL[l]);
     }
-    rec[1 + 3 * ND] = index_bits(v.nb, 0.0);
-    if(ER > 2 + 3 * ND) rec[ER - 1] = 0.0;
+    bool zero = true;
+#pragma unroll
+    for(int l = 0; l < ND; l++) zero &= v.rRL[l] == 0.0;
+    wide |= zero;
+    rec[RL::A] = v.area;
+    rec[RL::NB] = __longlong_as_double((long long)(((uint64_t)wide << 32) | (uint32_t)v.nb));
+    if(ND == 3) rec[entry_rec(ND, false) - 1] = 0.0;
 }
 template <int ND>
 __device__ __forceinline__ void entry_record_f64(const MeshView<double>& m, int32_t e,
@@ -1113,11 +1153,19 @@ __device__ __forceinline__ void grad_cell_f32(const MeshView<float>& m, int64_t 
     }
 }
 
+// The FP64 (parity) gradients.  In 3D bound by the records' bytes: 250,000
+// Poisson cells read 96 + 32 bytes of records an entry, 500 MB with padding,
+// 146 us; chunks of 1 to 3 records, limiter chunks of 4 to 8 and 3 or 4 waves
+// per SIMD are within 3%.  With IEEE quotients (30 divides a face, two a
+// limiter candidate, 480 of 900 instructions) and the limiter reading 48
+// bytes an entry it took 188 us, and 38 where 2D takes 26 us (150,001 cells).
 // Cell i; its gradients go to grad[(i + gshift) * ND * NC ...] (gshift: 0
 // for a whole mesh, the arena offset of the cell's mesh in an ensemble).
-template <int ND, typename T, typename R, bool DIFF, bool GROUPED, bool ACT>
+template <int ND, typename T, bool GROUPED, bool ACT>
 __device__ __forceinline__ void grad_cell_f64(const MeshView<T>& m, int64_t s,
                                               T* __restrict__ grad, int64_t gshift) {
+    using R = double;
+    using RL = Rec64<ND>;
     constexpr int NC = ND + 2, ER = entry_rec<ND, T>();
     // slot s (as in grad_cell_f32); the loads that depend on nothing go out
     // together: the record range and the slot's cell, then the activity
@@ -1141,6 +1189,9 @@ __device__ __forceinline__ void grad_cell_f64(const MeshView<T>& m, int64_t s,
         for(int l = 0; l < ND; l++) delta[l][k] = R(0);
     }
     const R V = (R)m.volume[i];
+    bool ieee = false;  // an operand out of quot_by's range
+#pragma unroll
+    for(int k = 0; k < NC; k++) ieee |= quot_wide(W[k]);
     if(!act) n = 0;
     // the cell's records as positions n - 1 .. 0 (reverse walk order,
     // src/VorCell.cpp:471): entries base + p, or rows base + p of the
@@ -1156,18 +1207,20 @@ __device__ __forceinline__ void grad_cell_f64(const MeshView<T>& m, int64_t s,
     for(int64_t pb = n; pb > 0; pb -= KB) {
         R A[KB], c[KB][ND], rij[KB][ND], Wj[KB][NC];
         int32_t o[KB];
+        bool wide[KB];
 #pragma unroll
         for(int u = 0; u < KB; u++) {
             const int64_t p = pb - 1 - u;
             alignas(16) T rec[ER];
             load_record<ND, T, GROUPED>(m, base, p >= 0 ? p : 0, lane, rec);
-            A[u] = (R)rec[0];
+            A[u] = rec[RL::A];
 #pragma unroll
             for(int l = 0; l < ND; l++) {
-                c[u][l] = (R)rec[1 + l];
-                rij[u][l] = (R)rec[1 + ND + l];
+                c[u][l] = rec[RL::C + l];
+                rij[u][l] = rec[RL::R + l];
             }
-            o[u] = bits_index(rec[1 + 3 * ND]);
+            o[u] = bits_index(rec[RL::NB]);
+            wide[u] = (__double_as_longlong(rec[RL::NB]) >> 32) != 0;
         }
 #pragma unroll
         for(int u = 0; u < KB; u++) {
@@ -1194,23 +1247,53 @@ __device__ __forceinline__ void grad_cell_f64(const MeshView<T>& m, int64_t s,
                                      rij[u][ND - 1] * rij[u][ND - 1])
                               : sqrt(rij[u][0] * rij[u][0] + rij[u][1] * rij[u][1]);
 #pragma unroll
-            for(int l = ND; l--;) {
+            for(int k = 0; k < NC; k++) wide[u] |= quot_wide(Wj[u][k]);
+            ieee |= wide[u];
+            const Recip rn = recip_of(rnorm);
 #pragma unroll
-                for(int k = 0; k < NC; k++) {
-                    R t;
-                    if(DIFF)
-                        t = (Wj[u][k] - W[k]) * ((c[u][l] - R(0.5) * rij[u][l]) / rnorm);
-                    else
-                        t = (Wj[u][k] - W[k]) * c[u][l] / rnorm -
-                            R(0.5) * (W[k] + Wj[u][k]) * rij[u][l] / rnorm;
-                    delta[l][k] += A[u] * t;
-                }
-            }
+            for(int l = ND; l--;)
+#pragma unroll
+                for(int k = 0; k < NC; k++)
+                    delta[l][k] += A[u] * (quot_by((Wj[u][k] - W[k]) * c[u][l], rn) -
+                                           quot_by(R(0.5) * (W[k] + Wj[u][k]) * rij[u][l], rn));
 #pragma unroll
             for(int k = 0; k < NC; k++) {
                 Wmax[k] = smaxr<R>(Wmax[k], Wj[u][k]);
                 Wmin[k] = sminr<R>(Wmin[k], Wj[u][k]);
             }
+        }
+    }
+    if(ieee) {
+        // the sums again, a face at a time, with IEEE quotients
+#pragma unroll
+        for(int l = 0; l < ND; l++)
+#pragma unroll
+            for(int k = 0; k < NC; k++) delta[l][k] = R(0);
+        for(int64_t p = n - 1; p >= 0; p--) {
+            alignas(16) T rec[ER];
+            load_record<ND, T, GROUPED>(m, base, p, lane, rec);
+            if(!(rec[RL::A] != R(0))) continue;
+            const int32_t o = bits_index(rec[RL::NB]);
+            R Wj[NC], r2 = R(0);
+#pragma unroll
+            for(int k = 0; k < NC; k++) Wj[k] = m.W[(o >= 0 ? (int64_t)o : i) * NC + k];
+            if(o < 0) {
+                R rr[ND];
+#pragma unroll
+                for(int l = 0; l < ND; l++) rr[l] = -rec[RL::R + l];
+                mirror_velocity<ND, R>(Wj + 1, rr);
+            }
+#pragma unroll
+            for(int l = 0; l < ND; l++) r2 = l ? r2 + rec[RL::R + l] * rec[RL::R + l]
+                                               : rec[RL::R] * rec[RL::R];
+            const R rnorm = sqrt(r2);
+#pragma unroll
+            for(int l = ND; l--;)
+#pragma unroll
+                for(int k = 0; k < NC; k++)
+                    delta[l][k] += rec[RL::A] *
+                                   ((Wj[k] - W[k]) * rec[RL::C + l] / rnorm -
+                                    R(0.5) * (W[k] + Wj[k]) * rec[RL::R + l] / rnorm);
         }
     }
 #pragma unroll
@@ -1223,26 +1306,26 @@ __device__ __forceinline__ void grad_cell_f64(const MeshView<T>& m, int64_t s,
     // the limiter, KL records a time (their loads out together), same order
     constexpr int KL = 4;
     for(int64_t pb = n; pb > 0; pb -= KL) {
-        R Ah[KL], dd[KL][ND];
+        R dd[KL][ND];
 #pragma unroll
         for(int u = 0; u < KL; u++) {
             const int64_t p = pb - 1 - u;
             alignas(16) T rec[ER];
             load_record<ND, T, GROUPED>(m, base, p >= 0 ? p : 0, lane, rec);
-            Ah[u] = (R)rec[0];
 #pragma unroll
-            for(int l = 0; l < ND; l++) dd[u][l] = (R)rec[1 + 2 * ND + l];
+            for(int l = 0; l < ND; l++) dd[u][l] = rec[RL::D + l];
         }
 #pragma unroll
         for(int u = 0; u < KL; u++) {
-            if(u >= pb || !(Ah[u] != R(0))) continue;
+            if(u >= pb) continue;
 #pragma unroll
             for(int k = 0; k < NC; k++) {
                 R dp = delta[0][k] * dd[u][0] + delta[1][k] * dd[u][1];
                 if(ND == 3) dp += delta[ND - 1][k] * dd[u][ND - 1];
-                R q1 = (dp != R(0)) ? (Wmax[k] - W[k]) / dp : R(1);
-                R q2 = (dp != R(0)) ? (Wmin[k] - W[k]) / dp : R(1);
-                alpha[k] = sminr<R>(alpha[k], smaxr<R>(q1, q2));
+                // the larger of (Wmax - W)/dp and (Wmin - W)/dp: the one
+                // whose sides have the same sign
+                const R q = (dp != R(0)) ? (dp > R(0) ? Wmax[k] - W[k] : Wmin[k] - W[k]) / dp : R(1);
+                alpha[k] = sminr<R>(alpha[k], q);
             }
         }
     }
@@ -1289,14 +1372,14 @@ __device__ __forceinline__ void grad_cell(const MeshView<T>& m, int64_t s, T* __
     } else {
         if(m.egrp) {
             if(m.active)
-                grad_cell_f64<ND, T, R, DIFF, true, true>(m, s, grad, gshift);
+                grad_cell_f64<ND, T, true, true>(m, s, grad, gshift);
             else
-                grad_cell_f64<ND, T, R, DIFF, true, false>(m, s, grad, gshift);
+                grad_cell_f64<ND, T, true, false>(m, s, grad, gshift);
         } else {
             if(m.active)
-                grad_cell_f64<ND, T, R, DIFF, false, true>(m, s, grad, gshift);
+                grad_cell_f64<ND, T, false, true>(m, s, grad, gshift);
             else
-                grad_cell_f64<ND, T, R, DIFF, false, false>(m, s, grad, gshift);
+                grad_cell_f64<ND, T, false, false>(m, s, grad, gshift);
         }
     }
 }

@@ -330,10 +330,9 @@ class DeviceMesh:
     # within the group only stops the padding lanes from sharing cache lines
     # with their neighbours', while wider windows scatter a wave's cells and
     # with them its neighbour rows; FP64 gradients, whose records are read
-    # padding and all, 1.088 ms at 256 against 1.339 in cell order and 1.207
-    # at 1024; 512 moves 1.48x the gradients' unique bytes instead of 1.59x
-    # for 3.7% more time)
-    SORT_WINDOW = {"mixed": 64, "fp64": 512}
+    # padding and all, 250,000 Poisson cells in 3D: 146 us at 256, 151 at 192,
+    # 156 at 512, 162 at 1024 and 175 in cell order)
+    SORT_WINDOW = {"mixed": 64, "fp64": 256}
 
     def __init__(self, b, storage="fp64", device=None, grouped=None, face_records=None,
                  sort_window=None):
