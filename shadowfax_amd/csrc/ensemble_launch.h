@@ -25,7 +25,7 @@ hipError_t ens_step_impl(int ndim, int kind, const EnsArgs<T>& a, hipStream_t s)
         hipLaunchKernelGGL((ens::drain_gradients<ND, T, double, MIXED != 0>), gc, b, 0, s, a.m, \
                            a.grad, a.plan, grid);                                               \
         if(kind == 0)                                                                          \
-            with_root<MIXED == 0>(a.c, [&](auto root) {                                        \
+            with_root<true>(a.c, [&](auto root) {                                        \
                 hipLaunchKernelGGL((ens::drain_faces<ND, 0, MIXED, T, double,                  \
                                                      decltype(root)::value>),                  \
                                    gf, b, 0, s, a.m, a.grad, a.c, cf, a.dQL, a.fstatus, a.ctr, \
@@ -61,7 +61,7 @@ hipError_t ens_range_impl(int ndim, int kind, const EnsArgs<T>& a, int64_t cell0
                            a.grad, cell0, ncell, gshift);                                       \
         if(nface > 0) {                                                                        \
             if(kind == 0)                                                                      \
-                with_root<MIXED == 0>(a.c, [&](auto root) {                                    \
+                with_root<true>(a.c, [&](auto root) {                                    \
                     hipLaunchKernelGGL((ens::range_faces<ND, 0, MIXED, T, double,              \
                                                          decltype(root)::value>),              \
                                        gf, b, 0, s, a.m, a.grad, a.c, cf, a.dQL, a.fstatus,    \
@@ -95,7 +95,7 @@ hipError_t ens_queue_impl(int ndim, int kind, const EnsArgs<T>& a, const QueueAr
         fn = ndim == 3 ? (const void*)ens::queue_kernel<3, 1, MIXED, T, double, 0>
                        : (const void*)ens::queue_kernel<2, 1, MIXED, T, double, 0>;
     else
-        with_root<MIXED == 0>(a.c, [&](auto root) {
+        with_root<true>(a.c, [&](auto root) {
             constexpr int ROOT = decltype(root)::value;
             fn = ndim == 3 ? (const void*)ens::queue_kernel<3, 0, MIXED, T, double, ROOT>
                            : (const void*)ens::queue_kernel<2, 0, MIXED, T, double, ROOT>;

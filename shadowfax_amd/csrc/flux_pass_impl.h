@@ -1438,8 +1438,7 @@ __device__ __forceinline__ void load_grad(const T* grad, int64_t C, int64_t cell
 // The activity flag read for every cell of a mesh without an activity array.
 static __device__ const uint8_t kAllActive = 1;
 
-// ROOT: Consts::root of the FP64 exact solver (fp64::ex_solve; unused by the
-// others).  MIXED: 0 = FP64 parity solvers, 1 = mixed solvers (and, for a periodic
+// ROOT: Consts::root of the exact solvers (0 for HLLC).  MIXED: 0 = FP64 parity solvers, 1 = mixed solvers (and, for a periodic
 // face whose other copy has a lower index, no evaluation: the gather applies
 // that copy's flux with the opposite sign).
 // Face f: its flux goes to dQL[(f + qshift) * NC ...]; the gradients of its
@@ -1661,16 +1660,8 @@ __device__ __forceinline__ void face_item(const MeshView<T>& m, int64_t f,
                     wr64[k] = (double)WR[k];
                 }
                 if(KIND == 0) {
-                    float wlf[NC], wrf[NC], nf[ND];
-#pragma unroll
-                    for(int k = 0; k < NC; k++) {
-                        wlf[k] = (float)WL[k];
-                        wrf[k] = (float)WR[k];
-                    }
-#pragma unroll
-                    for(int l = 0; l < ND; l++) nf[l] = (float)n64[l];
-                    st |= mixed::exact_mixed<ND>(cf, cd, wlf, wrf, nf, !has_r, wl64, wr64, n64,
-                                                 v64, flux, iters, vac);
+                    st |= mixed::exact_mixed<ND, ROOT>(cf, cd, !has_r, wl64, wr64, n64, v64,
+                                                       flux, iters, vac);
                 } else {
                     st |= mixed::hllc_mixed<ND>(cf, cd, wl64, wr64, n64, v64, !has_r, flux,
                                                 vac);
@@ -1740,12 +1731,14 @@ __device__ __forceinline__ void face_item(const MeshView<T>& m, int64_t f,
     cnt[CNT_NFAIL] += fail;
 }
 
-// Waves per SIMD a face kernel is held to: the FP64 exact solver's
-// out-of-line general path would otherwise set the register count (244, two
-// waves; the kernel's own code needs 150 in 3D); the others as they come.
+// Waves per SIMD a face kernel is held to: the exact solvers' out-of-line
+// general paths would otherwise set the register count (244 and 161; the
+// kernels' own code needs 150 and 110 in 3D); the others as they come.
+// (Mixed exact faces, 250,000 3D cells: 89 us at 4, 102 at 3, 162 at 5,
+// spilling; 2D, 262,144 cells: 29.7 at 6, 30.4 at 5, 31.2 at 4.)
 template <int ND, int KIND, int MIXED>
 constexpr int face_waves() {
-    return KIND == 0 && MIXED == 0 ? (ND == 2 ? 4 : 3) : 1;
+    return KIND != 0 ? 1 : MIXED == 0 ? (ND == 2 ? 4 : 3) : (ND == 2 ? 6 : 4);
 }
 
 template <int ND, int KIND, int MIXED, typename T, typename R, bool FREC = false, int ROOT = 0>

@@ -74,22 +74,26 @@ hipError_t launch_face_fluxes<float>(int ndim, int kind, const flux::MeshView<fl
     if(m.F <= 0) return hipSuccess;
     const mixed::CF cf = mixed::make_cf(c);
     // with the per-face records, the variant that reads them
-#define SFX_FACE(ND, K)                                                                          \
-    do {                                                                                         \
-        if(m.frec)                                                                               \
-            hipLaunchKernelGGL((flux::face_flux_kernel<ND, K, 1, float, double, true>),          \
-                               grid_for(m.F, 256), dim3(256), 0, s, m, grad, c, cf, dQL, fstatus, \
-                               ctr);                                                             \
-        else                                                                                     \
-            hipLaunchKernelGGL((flux::face_flux_kernel<ND, K, 1, float, double>),                \
-                               grid_for(m.F, 256), dim3(256), 0, s, m, grad, c, cf, dQL, fstatus, \
-                               ctr);                                                             \
-    } while(0)
-    if(ndim == 3 && kind == 0) SFX_FACE(3, 0);
-    else if(ndim == 3) SFX_FACE(3, 1);
-    else if(kind == 0) SFX_FACE(2, 0);
-    else SFX_FACE(2, 1);
-#undef SFX_FACE
+    auto face = [&](auto nd, auto k) {
+        constexpr int ND = decltype(nd)::value, K = decltype(k)::value;
+        with_root<K == 0>(c, [&](auto root) {
+            constexpr int ROOT = decltype(root)::value;
+            if(m.frec)
+                hipLaunchKernelGGL((flux::face_flux_kernel<ND, K, 1, float, double, true, ROOT>),
+                                   grid_for(m.F, 256), dim3(256), 0, s, m, grad, c, cf, dQL,
+                                   fstatus, ctr);
+            else
+                hipLaunchKernelGGL((flux::face_flux_kernel<ND, K, 1, float, double, false, ROOT>),
+                                   grid_for(m.F, 256), dim3(256), 0, s, m, grad, c, cf, dQL,
+                                   fstatus, ctr);
+        });
+    };
+    const std::integral_constant<int, 0> exact;
+    const std::integral_constant<int, 1> hllc;
+    const std::integral_constant<int, 2> d2;
+    const std::integral_constant<int, 3> d3;
+    if(ndim == 3) kind == 0 ? face(d3, exact) : face(d3, hllc);
+    else kind == 0 ? face(d2, exact) : face(d2, hllc);
     return hipGetLastError();
 }
 

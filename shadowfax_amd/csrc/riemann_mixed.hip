@@ -8,8 +8,13 @@
 namespace sfx {
 namespace mixed {
 
-template <int ND, int KIND, typename T>
-__global__ __launch_bounds__(256) void solve_for_flux_kernel(
+#ifndef SFX_MIXED_WAVES  // waves per SIMD the exact kernels are held to (4M problems: 115 us;
+#define SFX_MIXED_WAVES 6  // 5: 124, 4: 128, 8, spilling: 134)
+#endif
+
+template <int ND, int KIND, typename T, int ROOT>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(ROOT != 0 ? SFX_MIXED_WAVES : 1, 10))) void solve_for_flux_kernel(
         CF c, Consts cd, int64_t N, const T* __restrict__ WL, const T* __restrict__ WR,
         const T* __restrict__ n, const T* __restrict__ v, const uint8_t* __restrict__ refl,
         T* __restrict__ F, uint8_t* __restrict__ status, unsigned long long* __restrict__ ctr) {
@@ -32,15 +37,7 @@ __global__ __launch_bounds__(256) void solve_for_flux_kernel(
         const bool r = refl ? refl[i] != 0 : false;
         uint8_t st;
         if(KIND == 0) {
-            float wl[NC], wr[NC], nn[ND];
-#pragma unroll
-            for(int k = 0; k < NC; k++) {
-                wl[k] = (float)wl64[k];
-                wr[k] = (float)wr64[k];
-            }
-#pragma unroll
-            for(int d = 0; d < ND; d++) nn[d] = (float)n64[d];
-            st = exact_mixed<ND>(c, cd, wl, wr, nn, r, wl64, wr64, n64, v64, f, iters, vac);
+            st = exact_mixed<ND, ROOT>(c, cd, r, wl64, wr64, n64, v64, f, iters, vac);
         } else {
             st = hllc_mixed<ND>(c, cd, wl64, wr64, n64, v64, r, f, vac);
         }
@@ -68,8 +65,69 @@ __global__ __launch_bounds__(256) void solve_for_flux_kernel(
 
 struct Straggler {
     int32_t i;
-    float p, lo, hi;
+    float p, lo, hi;  // the iterate (p, or z alone) and its bracket
     int32_t it;
+};
+
+// the two iterations' parts under one name
+template <int ND, int ROOT>
+struct Parts {
+    using Case = std::conditional_t<ROOT != 0, RootCase, ExactCase>;
+    static __device__ __forceinline__ void setup(const CF& c, const Consts& cd, bool refl,
+                                                 const double* WL, double* WR, const double* n,
+                                                 Case& s) {
+        if constexpr(ROOT != 0) {
+            root_setup<ND, ROOT>(c, cd, refl, WL, WR, n, s);
+        } else {
+            float wl[ND + 2], wr[ND + 2], nn[ND];
+#pragma unroll
+            for(int k = 0; k < ND + 2; k++) {
+                wl[k] = (float)WL[k];
+                wr[k] = (float)WR[k];
+            }
+#pragma unroll
+            for(int d = 0; d < ND; d++) nn[d] = (float)n[d];
+            exact_setup<ND>(c, cd, wl, wr, nn, refl, WL, WR, n, s);
+        }
+    }
+    static __device__ __forceinline__ void iterate(const CF& c, const Consts& cd, Case& s,
+                                                   int stop) {
+        if constexpr(ROOT != 0)
+            root_iterate<ROOT>(c, cd, s, stop);
+        else
+            exact_iterate(c, s, stop);
+    }
+    static __device__ __forceinline__ uint8_t finish(const CF& c, const Consts& cd, const Case& s,
+                                                     const double* WL, const double* WR,
+                                                     const double* n, const double* v, bool refl,
+                                                     double* F, unsigned& iters, unsigned& vac) {
+        if constexpr(ROOT != 0)
+            return root_finish<ND, ROOT>(c, cd, s, WL, WR, n, v, refl, F, iters, vac);
+        else
+            return exact_finish<ND>(c, cd, s, WL, WR, n, v, F, iters, vac);
+    }
+    static __device__ __forceinline__ void save(const Case& s, Straggler& g) {
+        if constexpr(ROOT != 0) {
+            g.p = s.z;
+            g.lo = g.hi = 0.f;
+        } else {
+            g.p = s.p;
+            g.lo = s.lo;
+            g.hi = s.hi;
+        }
+        g.it = s.it;
+    }
+    static __device__ __forceinline__ void restore(const Straggler& g, Case& s) {
+        if constexpr(ROOT != 0) {
+            s.z = g.p;
+        } else {
+            s.p = g.p;
+            s.lo = g.lo;
+            s.hi = g.hi;
+        }
+        s.it = g.it;
+        s.phase = EX_ITER;
+    }
 };
 
 constexpr int kSegs = 16;  // phase-1 segments per phase-2 block
@@ -78,26 +136,23 @@ template <int ND, typename T>
 __device__ __forceinline__ void load_problem(int64_t N, int64_t i, const T* __restrict__ WL,
                                              const T* __restrict__ WR, const T* __restrict__ n,
                                              const T* __restrict__ v, double* wl64, double* wr64,
-                                             double* n64, double* v64, float* wl, float* wr,
-                                             float* nn) {
+                                             double* n64, double* v64) {
     const int NC = ND + 2;
 #pragma unroll
     for(int k = 0; k < NC; k++) {
         wl64[k] = (double)WL[k * N + i];
         wr64[k] = (double)WR[k * N + i];
-        wl[k] = (float)wl64[k];
-        wr[k] = (float)wr64[k];
     }
 #pragma unroll
     for(int d = 0; d < ND; d++) {
         n64[d] = (double)n[d * N + i];
         v64[d] = v ? (double)v[d * N + i] : 0.0;
-        nn[d] = (float)n64[d];
     }
 }
 
-template <int ND, typename T>
-__global__ __launch_bounds__(256) void exact_phase1_kernel(
+template <int ND, typename T, int ROOT>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(ROOT != 0 ? SFX_MIXED_WAVES : 1, 10))) void exact_phase1_kernel(
         CF c, Consts cd, int64_t N, const T* __restrict__ WL, const T* __restrict__ WR,
         const T* __restrict__ n, const T* __restrict__ v, const uint8_t* __restrict__ refl,
         T* __restrict__ F, uint8_t* __restrict__ status, unsigned long long* __restrict__ ctr,
@@ -110,13 +165,15 @@ __global__ __launch_bounds__(256) void exact_phase1_kernel(
     const bool valid = i < N;
     unsigned iters = 0, vac = 0, fail = 0, done = 0;
     double wl64[NC], wr64[NC], n64[ND], v64[ND];
-    float wl[NC], wr[NC], nn[ND];
-    ExactCase s;
+    using X = Parts<ND, ROOT>;
+    typename X::Case s;
     s.phase = EX_DONE;
+    bool r = false;
     if(valid) {
-        load_problem<ND, T>(N, i, WL, WR, n, v, wl64, wr64, n64, v64, wl, wr, nn);
-        exact_setup<ND>(c, cd, wl, wr, nn, refl ? refl[i] != 0 : false, wl64, wr64, n64, s);
-        if(s.phase == EX_ITER) exact_iterate(c, s, stop);
+        load_problem<ND, T>(N, i, WL, WR, n, v, wl64, wr64, n64, v64);
+        r = refl ? refl[i] != 0 : false;
+        X::setup(c, cd, r, wl64, wr64, n64, s);
+        if(s.phase == EX_ITER) X::iterate(c, cd, s, stop);
     }
     const bool strag = valid && s.phase == EX_ITER;
     // slots in the block's segment: a ballot per wave, one LDS atomic per wave
@@ -129,14 +186,11 @@ __global__ __launch_bounds__(256) void exact_phase1_kernel(
         const unsigned slot = base + (unsigned)__popcll(mask & ((1ull << lane) - 1ull));
         Straggler g;
         g.i = (int32_t)i;
-        g.p = s.p;
-        g.lo = s.lo;
-        g.hi = s.hi;
-        g.it = s.it;
+        X::save(s, g);
         queue[(int64_t)blockIdx.x * blockDim.x + slot] = g;
     } else if(valid) {
         double f[NC];
-        const uint8_t st = exact_finish<ND>(c, cd, s, wl64, wr64, n64, v64, f, iters, vac);
+        const uint8_t st = X::finish(c, cd, s, wl64, wr64, n64, v64, r, f, iters, vac);
 #pragma unroll
         for(int k = 0; k < NC; k++) F[k * N + i] = (T)f[k];
         if(status) status[i] = st;
@@ -149,14 +203,16 @@ __global__ __launch_bounds__(256) void exact_phase1_kernel(
     block_add_counters(ctr, cv);
 }
 
-template <int ND, typename T>
-__global__ __launch_bounds__(256) void exact_phase2_kernel(
+template <int ND, typename T, int ROOT>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(ROOT != 0 ? SFX_MIXED_WAVES : 1, 10))) void exact_phase2_kernel(
         CF c, Consts cd, int64_t N, const T* __restrict__ WL, const T* __restrict__ WR,
         const T* __restrict__ n, const T* __restrict__ v, const uint8_t* __restrict__ refl,
         T* __restrict__ F, uint8_t* __restrict__ status, unsigned long long* __restrict__ ctr,
         const Straggler* __restrict__ queue, const unsigned* __restrict__ counts,
         int64_t nsegs) {
     const int NC = ND + 2;
+    using X = Parts<ND, ROOT>;
     __shared__ unsigned s_pre[kSegs + 1];
     const int64_t seg0 = (int64_t)blockIdx.x * kSegs;
     if(threadIdx.x == 0) {
@@ -176,17 +232,13 @@ __global__ __launch_bounds__(256) void exact_phase2_kernel(
         const Straggler g = queue[(seg0 + q) * blockDim.x + (k - s_pre[q])];
         const int64_t i = g.i;
         double wl64[NC], wr64[NC], n64[ND], v64[ND], f[NC];
-        float wl[NC], wr[NC], nn[ND];
-        load_problem<ND, T>(N, i, WL, WR, n, v, wl64, wr64, n64, v64, wl, wr, nn);
-        ExactCase s;
-        exact_setup<ND>(c, cd, wl, wr, nn, refl ? refl[i] != 0 : false, wl64, wr64, n64, s);
-        s.p = g.p;
-        s.lo = g.lo;
-        s.hi = g.hi;
-        s.it = g.it;
-        s.phase = EX_ITER;
-        exact_iterate(c, s, c.itmax);
-        const uint8_t st = exact_finish<ND>(c, cd, s, wl64, wr64, n64, v64, f, iters, vac);
+        load_problem<ND, T>(N, i, WL, WR, n, v, wl64, wr64, n64, v64);
+        const bool rf = refl ? refl[i] != 0 : false;
+        typename X::Case s;
+        X::setup(c, cd, rf, wl64, wr64, n64, s);
+        X::restore(g, s);
+        X::iterate(c, cd, s, c.itmax);
+        const uint8_t st = X::finish(c, cd, s, wl64, wr64, n64, v64, rf, f, iters, vac);
 #pragma unroll
         for(int r = 0; r < NC; r++) F[r * N + i] = (T)f[r];
         if(status) status[i] = st;
@@ -219,18 +271,20 @@ hipError_t launch_exact_mixed_split(int ndim, const Consts& c, int64_t N, const 
             (mixed::Straggler*)((char*)scratch + ((4 * nb + 255) / 256) * 256);
     const dim3 grid((unsigned)nb), block(256),
             grid2((unsigned)((nb + mixed::kSegs - 1) / mixed::kSegs));
-#define SFX_SPLIT(ND)                                                                          \
-    do {                                                                                       \
-        hipLaunchKernelGGL((mixed::exact_phase1_kernel<ND, T>), grid, block, 0, stream, cf, c, N, \
-                           WL, WR, n, v, refl, F, status, ctr, queue, counts, stop);            \
-        hipLaunchKernelGGL((mixed::exact_phase2_kernel<ND, T>), grid2, block, 0, stream, cf, c,  \
-                           N, WL, WR, n, v, refl, F, status, ctr, queue, counts, nb);           \
-    } while(0)
+    auto split = [&](auto nd) {
+        constexpr int ND = decltype(nd)::value;
+        with_root<true>(c, [&](auto root) {
+            constexpr int ROOT = decltype(root)::value;
+            hipLaunchKernelGGL((mixed::exact_phase1_kernel<ND, T, ROOT>), grid, block, 0, stream,
+                               cf, c, N, WL, WR, n, v, refl, F, status, ctr, queue, counts, stop);
+            hipLaunchKernelGGL((mixed::exact_phase2_kernel<ND, T, ROOT>), grid2, block, 0, stream,
+                               cf, c, N, WL, WR, n, v, refl, F, status, ctr, queue, counts, nb);
+        });
+    };
     if(ndim == 3)
-        SFX_SPLIT(3);
+        split(std::integral_constant<int, 3>());
     else
-        SFX_SPLIT(2);
-#undef SFX_SPLIT
+        split(std::integral_constant<int, 2>());
     return hipGetLastError();
 }
 
@@ -254,14 +308,20 @@ hipError_t launch_solve_for_flux_mixed(int kind, int ndim, const Consts& c, int6
     const mixed::CF cf = mixed::make_cf(c);
     const int bs = 256;
     dim3 grid((unsigned)((N + bs - 1) / bs)), block(bs);
-#define SFX_LAUNCH(ND, K)                                                                 \
-    hipLaunchKernelGGL((mixed::solve_for_flux_kernel<ND, K, T>), grid, block, 0, stream, cf, \
-                       c, N, WL, WR, n, v, refl, F, status, ctr)
-    if(ndim == 3 && kind == 0) SFX_LAUNCH(3, 0);
-    else if(ndim == 3) SFX_LAUNCH(3, 1);
-    else if(kind == 0) SFX_LAUNCH(2, 0);
-    else SFX_LAUNCH(2, 1);
-#undef SFX_LAUNCH
+    auto solve = [&](auto nd, auto k) {
+        constexpr int ND = decltype(nd)::value, K = decltype(k)::value;
+        with_root<K == 0>(c, [&](auto root) {
+            hipLaunchKernelGGL((mixed::solve_for_flux_kernel<ND, K, T, decltype(root)::value>),
+                               grid, block, 0, stream, cf, c, N, WL, WR, n, v, refl, F, status,
+                               ctr);
+        });
+    };
+    const std::integral_constant<int, 0> exact;
+    const std::integral_constant<int, 1> hllc;
+    const std::integral_constant<int, 2> d2;
+    const std::integral_constant<int, 3> d3;
+    if(ndim == 3) kind == 0 ? solve(d3, exact) : solve(d3, hllc);
+    else kind == 0 ? solve(d2, exact) : solve(d2, hllc);
     return hipGetLastError();
 }
 

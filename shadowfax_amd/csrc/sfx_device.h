@@ -20,7 +20,7 @@ struct Consts {
     double tol, cutoff;
     int itercap;   // bound on Newton and on Brent iterations (reference: none)
     int fast53;    // gamma == 5/3: exponents 0.2, 0.6, 0.8, 3, 5 (mixed path)
-    // FP64 exact solver: 2 gamma/(gamma-1) where that is 5 (gamma = 5/3) or 7
+    // exact solvers: 2 gamma/(gamma-1) where that is 5 (gamma = 5/3) or 7
     // (gamma = 7/5), else 0; 1/root and (1 + 1/root)/(2 root), its root
     // series; sqrt(2/(gamma (gamma+1)))
     int root;
@@ -29,7 +29,7 @@ struct Consts {
 };
 
 // f(std::integral_constant<int, ROOT>) for the kernels that take Consts::root
-// as a template parameter: the FP64 exact solver's (exact), 0 for all others
+// as a template parameter: the exact solvers' (exact), 0 for HLLC's
 template <bool exact, class Fn>
 inline void with_root(const Consts& c, Fn f) {
     if constexpr(exact) {
