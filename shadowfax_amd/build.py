@@ -43,6 +43,9 @@ SOURCES = [
     ("mesh_voronoi3d.cpp", ["-ffp-contract=off"]),
     ("ensemble_fp64.hip", ["-ffp-contract=off"]),
     ("ensemble_mixed.hip", ["-ffp-contract=on", "-fno-hip-fp32-correctly-rounded-divide-sqrt"]),
+    ("ensemble_queue_fp64.hip", ["-ffp-contract=off"]),
+    ("ensemble_queue_mixed.hip", ["-ffp-contract=on",
+                                  "-fno-hip-fp32-correctly-rounded-divide-sqrt"]),
     ("sfx_ensemble.cpp", []),
     ("snapshot_hdf5.cpp", []),
 ]

@@ -1,0 +1,15 @@
+// ensemble_queue_fp64.hip -- the persistent serving kernel of the FP64 ensembles,
+// in a translation unit of its own (it is the longest to compile), with the
+// flags of the standalone flux pass of that precision.
+#include "ensemble_queue_launch.h"
+
+namespace sfx {
+
+template <>
+hipError_t ens_launch_queue<double>(int ndim, int kind, const EnsArgs<double>& a, const QueueArgs& qa,
+                                int ncu, hipStream_t s, int* blocks) {
+    return ens_queue_impl<double, 0>(ndim, kind, a, qa, ncu, s, blocks);
+}
+
+
+}  // namespace sfx
