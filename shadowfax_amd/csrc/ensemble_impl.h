@@ -196,8 +196,7 @@ __global__ __launch_bounds__(256) void drain_update(Consts cd, double* __restric
     drain<false>(p, 3, grid, [&](const Slot&, int64_t i) {
         fail += flux::update_cell<ND>(cd, i, Q, dQ, volume, W, cstatus, mass);
     });
-    const unsigned cv[CNT_N] = {0u, 0u, 0u, 0u, fail};
-    block_add_counters(ctr, cv);
+    wave_add_counter(ctr, CNT_NFAIL, fail);
 }
 
 // ---- one mesh, plain launches sized to the mesh (the unbatched path) ----
@@ -252,8 +251,7 @@ __global__ __launch_bounds__(256) void range_update(Consts cd, double* __restric
     const int64_t k = xcd_block() * blockDim.x + threadIdx.x;
     unsigned fail = 0;
     if(k < ncell) fail = flux::update_cell<ND>(cd, cell0 + k, Q, dQ, volume, W, cstatus, mass);
-    const unsigned cv[CNT_N] = {0u, 0u, 0u, 0u, fail};
-    block_add_counters(ctr, cv);
+    wave_add_counter(ctr, CNT_NFAIL, fail);
 }
 
 }  // namespace ens

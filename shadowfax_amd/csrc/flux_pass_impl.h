@@ -2039,8 +2039,7 @@ __global__ __launch_bounds__(256) void update_kernel(Consts cd, int64_t C, doubl
         const bool rebuild = endtime ? endtime[i] == tnow : true;
         fail = update_cell<ND>(cd, i, Q, dQ, volume, Wout, cstatus, mass, rebuild);
     }
-    const unsigned cv[CNT_N] = {0u, 0u, 0u, 0u, fail};
-    block_add_counters(ctr, cv);
+    wave_add_counter(ctr, CNT_NFAIL, fail);
 }
 
 }  // namespace flux
