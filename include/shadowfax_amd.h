@@ -577,6 +577,9 @@ int sfx_ensemble_step_plain(sfx_ensemble* e, int32_t id);
 int sfx_ensemble_sync(sfx_ensemble* e);
 /* Copies W, Q or dQ (SFX_ENS_*) of one mesh to host_out ([C][ndim+2]). */
 int sfx_ensemble_read(sfx_ensemble* e, int32_t id, int what, double* host_out);
+/* The same component-major, [ndim+2][C] (a small mesh's values in half the
+ * time: no runtime copy is involved). */
+int sfx_ensemble_read_components(sfx_ensemble* e, int32_t id, int what, double* host_out);
 
 /* Launch shape of the batched step's kernels: threads per block (= cells
  * or faces per work tile; 64..256, a multiple of 64) and blocks per CU of

@@ -311,6 +311,10 @@ hipError_t ens_launch_queue(int ndim, int kind, const EnsArgs<T>& a, const Queue
 hipError_t ens_launch_plan(const int32_t* batch, const int64_t* mcell0, const int64_t* mncell,
                            const int64_t* mface0, const int64_t* mnface, int32_t tile,
                            ens::Plan* plan, hipStream_t s);
+// dst[f - f0] = src[i nc + k], f = k n + i, for f0 <= f < f0 + count; dst may be
+// pinned host memory
+hipError_t ens_launch_components(const double* src, double* dst, int64_t f0, int64_t count,
+                                 int64_t n, int nc, hipStream_t s);
 hipError_t ens_launch_offset_i32(const int32_t* src, int32_t* dst, int64_t n, int64_t off,
                                  hipStream_t s);
 hipError_t ens_launch_offset_i64(const int64_t* src, int64_t* dst, int64_t n, int64_t off,

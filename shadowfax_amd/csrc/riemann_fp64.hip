@@ -92,9 +92,64 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void e
     block_add_counters(ctr, cv);
 }
 
+// One lane solves one problem (see ScalarIn).
+template <int ND, int KIND, int ROOT, bool SOLVE>
+__global__ __launch_bounds__(64) void scalar_kernel(Consts c, ScalarIn in,
+                                                    ScalarOut* __restrict__ out,
+                                                    unsigned long long* __restrict__ ctr) {
+    if(threadIdx.x) return;
+    unsigned iters = 0, brent = 0, vac = 0;
+    double f[ND + 2], mach = in.mach;
+    uint8_t st;
+    if constexpr(SOLVE) {
+        st = ex_solve<ND, ROOT>(c, in.WL, in.WR, in.n, in.reflective != 0, f, &mach, iters, brent,
+                                vac);
+    } else if constexpr(KIND == 0) {
+        st = ex_solve_for_flux<ND, ROOT>(c, in.WL, in.WR, in.n, in.v, in.reflective != 0, f, iters,
+                                         brent, vac);
+    } else {
+        st = hllc_solve_for_flux<ND>(c, in.WL, in.WR, in.n, in.v, in.reflective != 0, f, vac);
+    }
+    const unsigned cv[CNT_N] = {1u, brent, vac, iters, st != 0};
+    lane_add_counters(ctr, cv);
+#pragma unroll
+    for(int k = 0; k < ND + 2; k++) out->out[k] = f[k];
+    out->mach = mach;
+    out->status = st;
+    // everything above is on its way before the host sees the number
+    __hip_atomic_store(&out->seq, in.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 }  // namespace fp64
 
 // ------------------------------------------------------------ launchers --
+
+hipError_t launch_scalar_fp64(int kind, int ndim, bool solve_only, const Consts& c,
+                              const ScalarIn& in, ScalarOut* out, unsigned long long* ctr,
+                              hipStream_t stream) {
+    auto run = [&](auto nd) {
+        constexpr int ND = decltype(nd)::value;
+        if(kind != 0) {
+            hipLaunchKernelGGL((fp64::scalar_kernel<ND, 1, 0, false>), dim3(1), dim3(64), 0, stream,
+                               c, in, out, ctr);
+            return;
+        }
+        with_root<true>(c, [&](auto root) {
+            constexpr int ROOT = decltype(root)::value;
+            if(solve_only)
+                hipLaunchKernelGGL((fp64::scalar_kernel<ND, 0, ROOT, true>), dim3(1), dim3(64), 0,
+                                   stream, c, in, out, ctr);
+            else
+                hipLaunchKernelGGL((fp64::scalar_kernel<ND, 0, ROOT, false>), dim3(1), dim3(64), 0,
+                                   stream, c, in, out, ctr);
+        });
+    };
+    if(ndim == 3)
+        run(std::integral_constant<int, 3>());
+    else
+        run(std::integral_constant<int, 2>());
+    return hipGetLastError();
+}
 
 static inline unsigned nblocks(int64_t N, int bs) { return (unsigned)((N + bs - 1) / bs); }
 

@@ -50,6 +50,30 @@ __attribute__((amdgpu_waves_per_eu(ROOT != 0 ? SFX_MIXED_WAVES : 1, 10))) void s
     block_add_counters(ctr, cv);
 }
 
+// One lane solves one problem (see ScalarIn).
+template <int ND, int KIND, int ROOT>
+__global__ __launch_bounds__(64) void scalar_kernel(CF c, Consts cd, ScalarIn in,
+                                                    ScalarOut* __restrict__ out,
+                                                    unsigned long long* __restrict__ ctr) {
+    if(threadIdx.x) return;
+    unsigned iters = 0, vac = 0;
+    double f[ND + 2];
+    uint8_t st;
+    if constexpr(KIND == 0)
+        st = exact_mixed<ND, ROOT>(c, cd, in.reflective != 0, in.WL, in.WR, in.n, in.v, f, iters,
+                                   vac);
+    else
+        st = hllc_mixed<ND>(c, cd, in.WL, in.WR, in.n, in.v, in.reflective != 0, f, vac);
+    const unsigned cv[CNT_N] = {1u, 0u, vac, iters, st != 0};
+    lane_add_counters(ctr, cv);
+#pragma unroll
+    for(int k = 0; k < ND + 2; k++) out->out[k] = f[k];
+    out->mach = in.mach;
+    out->status = st;
+    // everything above is on its way before the host sees the number
+    __hip_atomic_store(&out->seq, in.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ---- exact solver in two phases (wave-level compaction) -----------------
 //
 // Phase 1 runs every problem's setup and at most `stop` FP32 Newton
@@ -250,6 +274,27 @@ __attribute__((amdgpu_waves_per_eu(ROOT != 0 ? SFX_MIXED_WAVES : 1, 10))) void e
 }
 
 }  // namespace mixed
+
+hipError_t launch_scalar_mixed(int kind, int ndim, const Consts& c, const ScalarIn& in,
+                               ScalarOut* out, unsigned long long* ctr, hipStream_t stream) {
+    const mixed::CF cf = mixed::make_cf(c);
+    auto run = [&](auto nd) {
+        constexpr int ND = decltype(nd)::value;
+        if(kind != 0)
+            hipLaunchKernelGGL((mixed::scalar_kernel<ND, 1, 0>), dim3(1), dim3(64), 0, stream, cf, c,
+                               in, out, ctr);
+        else
+            with_root<true>(c, [&](auto root) {
+                hipLaunchKernelGGL((mixed::scalar_kernel<ND, 0, decltype(root)::value>), dim3(1),
+                                   dim3(64), 0, stream, cf, c, in, out, ctr);
+            });
+    };
+    if(ndim == 3)
+        run(std::integral_constant<int, 3>());
+    else
+        run(std::integral_constant<int, 2>());
+    return hipGetLastError();
+}
 
 size_t exact_split_scratch_bytes(int64_t N) {
     const int64_t nb = (std::max<int64_t>(N, 1) + 255) / 256;

@@ -7,7 +7,9 @@
 
 #include "sfx_device.h"
 
-constexpr int kStageDoubles = 24;
+namespace sfx {
+struct ScalarOut;
+}
 
 struct sfx_solver {
     int kind = 0;
@@ -17,8 +19,9 @@ struct sfx_solver {
     sfx::Consts c{};
     bool stats_on = true;
     unsigned long long* d_ctr = nullptr;  // CNT_N device counters
-    double* d_stage = nullptr;            // scalar entry points: device staging
-    double* h_stage = nullptr;            // pinned host staging
+    sfx::ScalarOut* h_out = nullptr;      // scalar entry points: the result,
+    sfx::ScalarOut* d_out = nullptr;      // pinned, and as the device sees it
+    unsigned seq = 0;                     // the last scalar call's number
     // work buffer (the straggler queue of the two-phase exact solve), grown
     // on demand
     void* d_scratch = nullptr;

@@ -104,6 +104,15 @@ __device__ __forceinline__ void wave_add_counter(unsigned long long* ctr, int k,
         atomicAdd(ctr + (blockIdx.x % kCtrSlots) * CNT_N + k, s);
 }
 
+// One lane's counters, to slot 0.
+__device__ __forceinline__ void lane_add_counters(unsigned long long* ctr,
+                                                  const unsigned (&v)[CNT_N]) {
+    if(!ctr) return;
+#pragma unroll
+    for(int k = 0; k < CNT_N; k++)
+        if(v[k]) atomicAdd(ctr + k, (unsigned long long)v[k]);
+}
+
 // Workgroups are dispatched to the 8 XCDs of an MI355X round-robin
 // (dispatch index b runs on XCD b % 8) and every XCD has its own L2.  This
 // maps the dispatch index to a logical block index such that each XCD works

@@ -9,6 +9,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 #include <thread>
 #include <vector>
 
@@ -18,6 +19,8 @@
 #include "shadowfax_amd.h"
 
 using namespace sfx;
+
+constexpr int64_t kReadValues = 1 << 17;
 
 struct sfx_ensemble {
     sfx_solver* h = nullptr;
@@ -53,6 +56,9 @@ struct sfx_ensemble {
     void* dQL = nullptr;
     // batching
     int32_t* h_batch = nullptr;  // pinned [1 + kMaxBatch]
+    // pinned, written by the kernel that reads a mesh back
+    double *h_read = nullptr, *d_read = nullptr;  // [kReadValues]
+    std::mutex read_mu;                           // held by the read that uses it
     int32_t* d_batch = nullptr;
     ens::Plan* d_plan = nullptr;
     hipStream_t stream = nullptr;
@@ -72,6 +78,7 @@ int ens_free(sfx_ensemble* e) {
     if(e->graph) hipGraphDestroy(e->graph);
     for(void* p : e->allocs) hipFree(p);
     if(e->h_batch) hipHostFree(e->h_batch);
+    if(e->h_read) hipHostFree(e->h_read);
     if(e->stream) hipStreamDestroy(e->stream);
     delete e;
     return SFX_OK;
@@ -489,6 +496,10 @@ int sfx_ensemble_create(sfx_solver* h, int64_t max_meshes, int64_t max_cells, in
     e->egeo_bytes = std::max<size_t>(t * E * ER, 256);
     if(err == hipSuccess) err = hipHostMalloc((void**)&e->h_batch,
                                               sizeof(int32_t) * (1 + ens::kMaxBatch));
+    if(err == hipSuccess)
+        err = hipHostMalloc((void**)&e->h_read, 8 * kReadValues,
+                            hipHostMallocMapped | hipHostMallocCoherent);
+    if(err == hipSuccess) err = hipHostGetDevicePointer((void**)&e->d_read, e->h_read, 0);
     if(err == hipSuccess) err = hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking);
     if(err == hipSuccess) err = hipMemsetAsync(e->dQ, 0, 8 * C * NC, e->stream);
     if(err == hipSuccess) err = hipStreamSynchronize(e->stream);
@@ -661,20 +672,52 @@ int sfx_ensemble_sync(sfx_ensemble* e) {
     return err == hipSuccess ? SFX_OK : hip_error(err, "sfx_ensemble_sync");
 }
 
-int sfx_ensemble_read(sfx_ensemble* e, int32_t id, int what, double* host_out) {
-    if(!e || !host_out) return set_error(SFX_ERR_ARG, "sfx_ensemble_read: NULL");
-    if(id < 0 || id >= e->nmesh) return set_error(SFX_ERR_ARG, "sfx_ensemble_read: id");
+// the device rows of mesh id's W, Q or dQ; null (with the error set) if none
+static const double* read_source(sfx_ensemble* e, int32_t id, int what, const double* host_out) {
+    if(!e || !host_out) {
+        set_error(SFX_ERR_ARG, "sfx_ensemble_read: NULL");
+        return nullptr;
+    }
+    if(id < 0 || id >= e->nmesh) {
+        set_error(SFX_ERR_ARG, "sfx_ensemble_read: id");
+        return nullptr;
+    }
     const double* src = what == SFX_ENS_W ? e->W : what == SFX_ENS_Q ? e->Q : what == SFX_ENS_DQ
                                                                                   ? e->dQ
                                                                                   : nullptr;
-    if(!src) return set_error(SFX_ERR_ARG, "sfx_ensemble_read: what");
+    if(!src) {
+        set_error(SFX_ERR_ARG, "sfx_ensemble_read: what");
+        return nullptr;
+    }
+    return src + e->c0[id] * e->NC;
+}
+
+int sfx_ensemble_read(sfx_ensemble* e, int32_t id, int what, double* host_out) {
+    const double* src = read_source(e, id, what, host_out);
+    if(!src) return SFX_ERR_ARG;
     int rc = bind_device(e->h);
     if(rc) return rc;
     hipError_t err = hipStreamSynchronize(e->stream);
     if(err == hipSuccess)
-        err = hipMemcpy(host_out, src + e->c0[id] * e->NC, 8 * e->nc[id] * e->NC,
-                        hipMemcpyDeviceToHost);
+        err = hipMemcpy(host_out, src, 8 * e->nc[id] * e->NC, hipMemcpyDeviceToHost);
     return err == hipSuccess ? SFX_OK : hip_error(err, "sfx_ensemble_read");
+}
+
+int sfx_ensemble_read_components(sfx_ensemble* e, int32_t id, int what, double* host_out) {
+    const double* src = read_source(e, id, what, host_out);
+    if(!src) return SFX_ERR_ARG;
+    int rc = bind_device(e->h);
+    if(rc) return rc;
+    const int64_t n = e->nc[id], all = n * e->NC;
+    std::lock_guard<std::mutex> lk(e->read_mu);
+    hipError_t err = hipSuccess;
+    for(int64_t f0 = 0; f0 < all && err == hipSuccess; f0 += kReadValues) {
+        const int64_t m = std::min(all - f0, kReadValues);
+        err = ens_launch_components(src, e->d_read, f0, m, n, e->NC, e->stream);
+        if(err == hipSuccess) err = hipStreamSynchronize(e->stream);
+        if(err == hipSuccess) std::memcpy(host_out + f0, e->h_read, 8 * (size_t)m);
+    }
+    return err == hipSuccess ? SFX_OK : hip_error(err, "sfx_ensemble_read_components");
 }
 
 int sfx_ensemble_set_launch(sfx_ensemble* e, int block, int blocks_per_cu) {

@@ -20,6 +20,24 @@ hipError_t launch_exact_solve_fp64(int ndim, const Consts& c, int64_t N, const d
                                    double* Whalf, double* WRout, double* mach, uint8_t* status,
                                    unsigned long long* ctr, hipStream_t stream);
 
+// One problem, its values among the kernel's arguments, its result written
+// straight to host memory (pinned, coherent): status and, last, seq.
+struct ScalarIn {
+    double WL[5], WR[5], n[3], v[3], mach;
+    int reflective;
+    uint32_t seq;
+};
+struct ScalarOut {
+    double out[5], mach;
+    uint32_t status, seq;
+};
+// solve_only: ExactRiemannSolver::solve (half state and Mach number)
+hipError_t launch_scalar_fp64(int kind, int ndim, bool solve_only, const Consts& c,
+                              const ScalarIn& in, ScalarOut* out, unsigned long long* ctr,
+                              hipStream_t stream);
+hipError_t launch_scalar_mixed(int kind, int ndim, const Consts& c, const ScalarIn& in,
+                               ScalarOut* out, unsigned long long* ctr, hipStream_t stream);
+
 // riemann_mixed.hip: T = float (FP32 storage) or double (FP64 storage)
 template <typename T>
 hipError_t launch_solve_for_flux_mixed(int kind, int ndim, const Consts& c, int64_t N,

@@ -48,6 +48,7 @@ def _lib():
         L.sfx_ensemble_step_plain.argtypes = [vp, i32]
         L.sfx_ensemble_sync.argtypes = [vp]
         L.sfx_ensemble_read.argtypes = [vp, i32, ct.c_int, _dp]
+        L.sfx_ensemble_read_components.argtypes = [vp, i32, ct.c_int, _dp]
         L.sfx_ensemble_set_launch.argtypes = [vp, ct.c_int, ct.c_int]
         L.sfx_ensemble_get_launch.argtypes = [vp, ct.POINTER(ct.c_int), ct.POINTER(ct.c_int)]
         L.sfx_ensemble_autotune.argtypes = [vp, _i32p, i32, ct.c_int, _dp]
@@ -126,10 +127,10 @@ class Ensemble:
 
     def read(self, mid, what=ENS_W):
         """W, Q or dQ of one mesh, component-major (ndim+2, C)."""
-        out = np.zeros((self.cells[mid], self.ndim + 2))
-        Cp.check(_lib().sfx_ensemble_read(self.h, int(mid), what, _p(out, _dp)),
-                 "sfx_ensemble_read")
-        return out.T.copy()
+        out = np.empty((self.ndim + 2, self.cells[mid]))
+        Cp.check(_lib().sfx_ensemble_read_components(self.h, int(mid), what, _p(out, _dp)),
+                 "sfx_ensemble_read_components")
+        return out
 
     def set_launch(self, block, blocks_per_cu):
         Cp.check(_lib().sfx_ensemble_set_launch(self.h, block, blocks_per_cu),
