@@ -325,9 +325,19 @@ __device__ __forceinline__ float quot_r<float>(float a, float b) {
 // get_time_derivative (ExactRiemannSolver.cpp:892-934 / HLLCRiemannSolver.cpp:
 // 415-450); g[d][k] = dW_k/dx_d.  The 2D dWdt[2] uses gradients[1].vy()
 // twice, as the reference does (:920 / :443).
-template <int ND, typename R>
+// ONE: the quotients by W[0] from one reciprocal (FP64, within half an ulp,
+// for W[0] and 1/W[0] in range; the face predictor), else quot_r.
+template <int ND, typename R, bool ONE = false>
 __device__ __forceinline__ void time_derivative(R gamma, const R* W, const R (*g)[ND + 2],
                                                 R* dWdt) {
+    R ir = R(0);
+    if constexpr(ONE) ir = fp64::rcp64(W[0]);
+    auto quot_r = [&](R a, R b) {
+        if constexpr(ONE)
+            return fp64::div_by(a, b, ir);
+        else
+            return flux::quot_r(a, b);
+    };
     if(ND == 3) {
         const R* gx = g[0];
         const R* gy = g[1];
@@ -348,32 +358,43 @@ __device__ __forceinline__ void time_derivative(R gamma, const R* W, const R (*g
     }
 }
 
-// VorFace::limit, scalar (src/VorFace.hpp:92-137); dnrm = |d| precomputed
-template <typename R>
-__device__ __forceinline__ R limit1(R phimid0, R phiL, R phiR, R dnrm, R r) {
-    const R psi1 = R(0.5), psi2 = R(0.25);
-    R delta1 = psi1 * fabs(phiL - phiR);
-    R delta2 = psi2 * fabs(phiL - phiR);
-    R phimin = rmin(phiL, phiR);
-    R phimax = rmax(phiL, phiR);
-    R phibar = phiL + dnrm / r * (phiR - phiL);
-    R phiplus = ((phimax + delta1) * phimax > R(0)) ? phimax + delta1
-                                                    : phimax / (R(1) + delta1 / fabs(phimax));
-    R phiminus = ((phimin - delta1) * phimin > R(0)) ? phimin - delta1
-                                                     : phimin / (R(1) + delta1 / fabs(phimin));
+// VorFace::limit, scalar (src/VorFace.hpp:92-137); t = |d|/r.  Only one of phi-
+// (phiL < phiR) and phi+ (phiL > phiR) is used, and the extremum it starts
+// from is phiL; phiL/(1 + delta1/|phiL|) as phiL (|phiL|/(|phiL| + delta1)),
+// one quotient instead of two (four with the unused one).
+__device__ __forceinline__ double limit1(double phimid0, double phiL, double phiR, double t) {
+    const double delta1 = 0.5 * fabs(phiL - phiR), delta2 = 0.25 * fabs(phiL - phiR);
+    const double phibar = phiL + t * (phiR - phiL);
+    const bool up = phiL < phiR;
+    const double far = up ? phiL - delta1 : phiL + delta1;
+    double lim = far;
+    if(!(far * phiL > 0.0)) {
+        const double a = fabs(phiL);
+        lim = phiL * fp64::div64(a, fmax(a + delta1, 1e-300));
+    }
     if(phiL == phiR) return phiL;
-    if(phiL < phiR) return rmax(phiminus, rmin(phibar + delta2, phimid0));
-    return rmin(phiplus, rmax(phibar - delta2, phimid0));
+    if(up) return rmax(lim, rmin(phibar + delta2, phimid0));
+    return rmin(lim, rmax(phibar - delta2, phimid0));
 }
 
-// One side of VorFace::calculate_flux's predictor (src/VorFace.cpp:714-804)
-template <int ND, typename R>
-__device__ __forceinline__ void predict_side(R gamma, const R* Wraw, const R* Wother,
-                                             const R (*g)[ND + 2], const R* d, R r,
-                                             bool limited, R dtp, R* out) {
+// One side of VorFace::calculate_flux's predictor (src/VorFace.cpp:714-804).
+// The FP64 face kernels are bound by instruction issue at 3 to 4 waves: with
+// the quotients of the predictor, the normal and the limiters from hardware
+// estimates (8 instructions, or 2 where the divisor is shared, for 12) and one
+// limiter quotient a component instead of four, 250,000 3D cells' pass takes
+// 315 us for 339, 150,000 2D cells' step 68.8 for 70.2.
+template <int ND>
+__device__ __forceinline__ void predict_side(double gamma, const double* Wraw,
+                                             const double* Wother, const double (*g)[ND + 2],
+                                             const double* d, double r, bool limited, double dtp,
+                                             double* out) {
+    using R = double;
     const int NC = ND + 2, P = ND + 1;
     R dWdt[NC], deltaW[NC], Wt[NC];
-    time_derivative<ND, R>(gamma, Wraw, g, dWdt);
+    if(Wraw[0] >= 1e-280 && Wraw[0] <= 1e280)
+        time_derivative<ND, R, true>(gamma, Wraw, g, dWdt);
+    else
+        time_derivative<ND, R>(gamma, Wraw, g, dWdt);
 #pragma unroll
     for(int k = 0; k < NC; k++) deltaW[k] = R(0.5) * dtp * dWdt[k];
     // VorFace::reconstruct (src/VorFace.hpp:174-196)
@@ -385,10 +406,11 @@ __device__ __forceinline__ void predict_side(R gamma, const R* Wraw, const R* Wo
             Wt[k] = Wraw[k] + (g[0][k] * d[0] + g[1][k] * d[1]);
     }
     if(limited) {
-        R dnrm = (ND == 3) ? sqrt(d[0] * d[0] + d[1] * d[1] + d[ND - 1] * d[ND - 1])
-                           : sqrt(d[0] * d[0] + d[1] * d[1]);
+        const R d2 = (ND == 3) ? d[0] * d[0] + d[1] * d[1] + d[ND - 1] * d[ND - 1]
+                               : d[0] * d[0] + d[1] * d[1];
+        const R t = sqrt(d2) / r;
 #pragma unroll
-        for(int k = 0; k < NC; k++) Wt[k] = limit1<R>(Wt[k], Wraw[k], Wother[k], dnrm, r);
+        for(int k = 0; k < NC; k++) Wt[k] = limit1(Wt[k], Wraw[k], Wother[k], t);
     }
     if(Wt[0] < R(0) || Wt[P] < R(0)) {
 #pragma unroll
@@ -1579,7 +1601,7 @@ __device__ __forceinline__ void face_item(const MeshView<T>& m, int64_t f,
                 if constexpr(MIXED)
                     fac *= mixed::rcp_nr(rRL2);
                 else
-                    fac /= rRL2;
+                    fac = fp64::div64(fac, rRL2);
 #pragma unroll
                 for(int l = 0; l < ND; l++) vface[l] = R(0.5) * (vl[l] + vr[l]) + fac * rr[l];
             } else {
@@ -1612,8 +1634,8 @@ __device__ __forceinline__ void face_item(const MeshView<T>& m, int64_t f,
                 if(has_r) predict_side_offset<ND>(gf, WR, WL, gR, dRs, rcf, true, dt, WRrec);
                 predict_side_offset<ND>(gf, WL, WR, gL, dLs, rcf, has_r, dt, WLrec);
             } else {
-                if(has_r) predict_side<ND, R>(gam, WR, WL, gR, dRf, rc, true, (R)dt, WRrec);
-                predict_side<ND, R>(gam, WL, WR, gL, dLf, rc, has_r, (R)dt, WLrec);
+                if(has_r) predict_side<ND>(gam, WR, WL, gR, dRf, rc, true, (R)dt, WRrec);
+                predict_side<ND>(gam, WL, WR, gL, dLf, rc, has_r, (R)dt, WLrec);
             }
             if(WL[0] != R(0)) {
 #pragma unroll
@@ -1629,9 +1651,10 @@ __device__ __forceinline__ void face_item(const MeshView<T>& m, int64_t f,
             double flux[NC];
             if(!MIXED) {
                 double n64[ND], v64[ND], wl[NC], wr[NC];
+                const double inrm = fp64::rcp64((double)nrm);
 #pragma unroll
                 for(int l = 0; l < ND; l++) {
-                    n64[l] = (double)(rr[l] / nrm);
+                    n64[l] = fp64::div_by((double)rr[l], (double)nrm, inrm);
                     v64[l] = (double)vface[l];
                 }
 #pragma unroll
@@ -1679,8 +1702,16 @@ __device__ __forceinline__ void face_item(const MeshView<T>& m, int64_t f,
                 areaL = m.total_area[L];
                 areaR = m.total_area[Rs];
             }
-            // the mixed pass takes its quotients through rcp_nr
+            // from reciprocals: a zero divisor gives NaN where a / b gives
+            // infinity, and no limit either way
             auto quot = [](double a, double b) {
+                if constexpr(MIXED)
+                    return a * mixed::rcp_nr(b);
+                else
+                    return fp64::div64(a, b);
+            };
+            // a flux may be of any size
+            auto quot_any = [](double a, double b) {
                 if constexpr(MIXED)
                     return a * mixed::rcp_nr(b);
                 else
@@ -1695,7 +1726,7 @@ __device__ __forceinline__ void face_item(const MeshView<T>& m, int64_t f,
             double areafac = quot((double)A, areaL);
             areafac *= timefac;
             if(dQ[0] > areafac * massL) {
-                double corfac = fabs(quot(areafac * massL, dQ[0]));
+                double corfac = fabs(quot_any(areafac * massL, dQ[0]));
 #pragma unroll
                 for(int k = 0; k < NC; k++) dQ[k] *= corfac;
             }
@@ -1704,7 +1735,7 @@ __device__ __forceinline__ void face_item(const MeshView<T>& m, int64_t f,
                 af *= timefac;
                 // dQR[0] = -dQL[0]
                 if(-dQ[0] > af * massR) {
-                    double corfac = fabs(quot(af * massR, -dQ[0]));
+                    double corfac = fabs(quot_any(af * massR, -dQ[0]));
 #pragma unroll
                     for(int k = 0; k < NC; k++) dQ[k] = -(-dQ[k] * corfac);
                 }

@@ -988,11 +988,11 @@ __device__ void hllc_vacuum_flux(const Consts& c, const double* WL, const double
     deboost<ND>(c, v, flux);
 }
 
-// HLLCRiemannSolver::solve_for_flux, HLLCRiemannSolver.cpp:258-403
+// HLLCRiemannSolver::solve_for_flux, HLLCRiemannSolver.cpp:258-403, expression
+// by expression: the path of the states that hllc_solve_for_flux does not take.
 template <int ND>
-__device__ uint8_t hllc_solve_for_flux(const Consts& c, const double* WL, double* WR,
-                                       const double* n, const double* v, bool reflective,
-                                       double* flux, unsigned& vac) {
+__device__ uint8_t hllc_steps(const Consts& c, const double* WL, double* WR, const double* n,
+                              const double* v, bool reflective, double* flux, unsigned& vac) {
     SFX_FP64_STRICT
     const int NC = S<ND>::NC, P = S<ND>::P;
     const double g = c.gamma;
@@ -1055,6 +1055,159 @@ __device__ uint8_t hllc_solve_for_flux(const Consts& c, const double* WL, double
 #pragma unroll
         for(int d = 0; d < ND; d++) flux[1 + d] += SK * (U[1 + d] - WK[0] * WK[1 + d]);
         flux[P] += SK * (U[P] - WK[0] * eK);
+    }
+    deboost<ND>(c, v, flux);
+    return 0;
+}
+
+template <int ND>
+struct HllcGeneral {
+    double WL[ND + 2], WR[ND + 2], n[ND], v[ND], F[ND + 2];
+    unsigned vac;
+    bool reflective;
+};
+template <int ND>
+__device__ __attribute__((noinline)) uint8_t hllc_general(Consts c, HllcGeneral<ND>* g) {
+    return hllc_steps<ND>(c, g->WL, g->WR, g->n, g->v, g->reflective, g->F, g->vac);
+}
+
+// solve_for_flux: the same expressions with quotients and roots from the
+// hardware's estimates (div64, sqrt64: within half an ulp, as the IEEE ones,
+// in 8 and 9 instructions instead of 12 and 22, shared where two quotients
+// have one divisor) and, for gamma 5/3 and 7/5, the vacuum fan's powers as
+// products.  States with a zero, negative, non-finite or extreme density or
+// pressure, or beyond Mach 1e12, go through hllc_steps, out of line.  1,048,576
+// 2D problems, 136 bytes each: 36.3 us expression by expression, 27.5 here
+// (5.2 TB/s, the rate of a copy).
+template <int ND>
+__device__ __forceinline__ uint8_t hllc_solve_for_flux(const Consts& c, const double* WL,
+                                                       double* WR, const double* n,
+                                                       const double* v, bool reflective,
+                                                       double* flux, unsigned& vac) {
+    SFX_FP64_STRICT
+    constexpr int NC = S<ND>::NC, P = S<ND>::P;
+    double uL = WL[1] * n[0] + WL[2] * n[1];
+    double uR = WR[1] * n[0] + WR[2] * n[1];
+    if(ND == 3) {
+        uL = WL[1] * n[0] + WL[2] * n[1] + WL[ND] * n[ND - 1];
+        uR = WR[1] * n[0] + WR[2] * n[1] + WR[ND] * n[ND - 1];
+    }
+    if(reflective) {
+#pragma unroll
+        for(int k = 0; k < NC; k++) WR[k] = WL[k];
+        uR = -uL;
+    }
+    const double rL = WL[0], pL = WL[P], rR = WR[0], pR = WR[P];
+    const double irL = rcp64(rL), irR = rcp64(rR), gm1 = c.gamma - 1., gm1inv = 0.5 * c.tdgm1;
+    const double aL = sqrt64(div_by(c.gamma * pL, rL, irL));
+    const double aR = sqrt64(div_by(c.gamma * pR, rR, irR));
+    // false for NaNs; within it no quotient below leaves the range of doubles
+    // and S_K - u_K is not rounded to zero
+    if(!(smin(rL, rR) >= 1e-50 && smin(pL, pR) >= 1e-50 && smax(rL, rR) <= 1e50 &&
+         smax(pL, pR) <= 1e50 && rR == rR && pR == pR &&
+         fabs(uL) <= 1e12 * smin(aL, aR) && fabs(uR) <= 1e12 * smin(aL, aR))) {
+        HllcGeneral<ND> g;
+#pragma unroll
+        for(int k = 0; k < NC; k++) {
+            g.WL[k] = WL[k];
+            g.WR[k] = WR[k];
+        }
+#pragma unroll
+        for(int d = 0; d < ND; d++) {
+            g.n[d] = n[d];
+            g.v[d] = v[d];
+        }
+        g.vac = vac;
+        g.reflective = reflective;
+        const uint8_t st = hllc_general<ND>(c, &g);
+#pragma unroll
+        for(int k = 0; k < NC; k++) flux[k] = g.F[k];
+        vac = g.vac;
+        return st;
+    }
+    bool left;
+    if(c.tdgm1 * aL + c.tdgm1 * aR <= uR - uL) {
+        // vacuum_flux between two gases (HLLCRiemannSolver.cpp:95-208)
+        vac = 1;
+        const double SR = uR - c.tdgm1 * aR, SL = uL + c.tdgm1 * aL;
+        left = SL >= 0.;
+        const bool none = SR > 0. && SL < 0., fan = left ? uL < aL : -uR < aR;
+        double sol[NC], vhalf = 0.;
+#pragma unroll
+        for(int k = 0; k < NC; k++) sol[k] = left ? WL[k] : WR[k];
+        if(none) {
+#pragma unroll
+            for(int k = 0; k < NC; k++) flux[k] = 0.;
+            return 0;
+        }
+        if(fan) {
+            const double sgn = left ? 1. : -1., aK = left ? aL : aR, uK = left ? uL : uR;
+            const double base = c.tdgp1 + div64(sgn * c.gm1dgp1 * uK, aK);
+            double fr, fp;
+            if(c.root == 5)
+                fan_powers<5>(c, base, fr, fp);
+            else if(c.root == 7)
+                fan_powers<7>(c, base, fr, fp);
+            else
+                fan_powers<0>(c, base, fr, fp);
+            sol[0] *= fr;
+            sol[P] *= fp;
+            vhalf = c.tdgp1 * (sgn * aK + c.gm1d2 * uK) - uK;
+        }
+#pragma unroll
+        for(int d = 0; d < ND; d++) sol[1 + d] += vhalf * n[d];
+#pragma unroll
+        for(int k = 0; k < NC; k++) flux[k] = 0.;
+        if(!(sol[0] != 0.)) return 0;
+        double vsol = sol[1] * n[0] + sol[2] * n[1];
+        double v2 = sol[1] * sol[1] + sol[2] * sol[2];
+        if(ND == 3) {
+            vsol += sol[ND] * n[ND - 1];
+            v2 += sol[ND] * sol[ND];
+        }
+        flux[0] = sol[0] * vsol;
+#pragma unroll
+        for(int d = 0; d < ND; d++) flux[1 + d] = sol[0] * sol[1 + d] * vsol + sol[P] * n[d];
+        // rho e = p/(g-1) + rho v^2/2: no quotient by a density that the fan
+        // may have made as small as it likes
+        flux[P] = (div_by(sol[P], gm1, gm1inv) + sol[0] * (0.5 * v2)) * vsol + sol[P] * vsol;
+        deboost<ND>(c, v, flux);
+        return 0;
+    }
+    const double rhobar = 0.5 * (rL + rR), abar = 0.5 * (aL + aR);
+    const double pstar = smax(0., 0.5 * (pL + pR) - 0.5 * (uR - uL) * rhobar * abar);
+    double qL = 1., qR = 1.;
+    if(pstar > pL) qL = sqrt64(1. + c.gp1d2g * (div64(pstar, pL) - 1.));
+    if(pstar > pR) qR = sqrt64(1. + c.gp1d2g * (div64(pstar, pR) - 1.));
+    const double SL = uL - aL * qL, SR = uR + aR * qR;
+    const double Sstar = div64(pR - pL + rL * uL * (SL - uL) - rR * uR * (SR - uR),
+                               rL * (SL - uL) - rR * (SR - uR));
+    left = Sstar >= 0.;
+    double W[NC];
+#pragma unroll
+    for(int k = 0; k < NC; k++) W[k] = left ? WL[k] : WR[k];
+    const double uK = left ? uL : uR, SK = left ? SL : SR, ir = left ? irL : irR;
+    flux[0] = W[0] * uK;
+#pragma unroll
+    for(int d = 0; d < ND; d++) flux[1 + d] = W[0] * W[1 + d] * uK + W[P] * n[d];
+    double v2 = W[1] * W[1] + W[2] * W[2];
+    if(ND == 3) v2 += W[ND] * W[ND];
+    const double eK = div_by(div_by(W[P], gm1, gm1inv), W[0], ir) + 0.5 * v2;
+    flux[P] = W[0] * eK * uK + W[P] * uK;
+    if(left ? (SK < 0.) : (SK > 0.)) {
+        const double du = Sstar - uK, m = W[0] * (SK - uK);
+        double U[NC];
+        U[0] = 1.;
+#pragma unroll
+        for(int d = 0; d < ND; d++) U[1 + d] = W[1 + d] + du * n[d];
+        U[P] = eK + du * (Sstar + div64(W[P], m));
+        const double fac = div64(m, SK - Sstar);
+#pragma unroll
+        for(int k = 0; k < NC; k++) U[k] *= fac;
+        flux[0] += SK * (U[0] - W[0]);
+#pragma unroll
+        for(int d = 0; d < ND; d++) flux[1 + d] += SK * (U[1 + d] - W[0] * W[1 + d]);
+        flux[P] += SK * (U[P] - W[0] * eK);
     }
     deboost<ND>(c, v, flux);
     return 0;
