@@ -407,7 +407,9 @@ int sfx_mesh_entry_record(int ndim, int precision);
 /* Per-face records of the mixed face pass (no counterpart in the reference:
  * a layout of the per-face values that VorFace::calculate_flux reads,
  * src/VorFace.cpp:670-760), built once per tessellation from the FP32 face
- * arrays of m: plane q of face f at float4 index q F + f,
+ * arrays of m: plane q of face f at float4 index P g + q n + f - g, g = f
+ * rounded down to a multiple of G = 4 (3D) or 8 (2D), n = min(G, F - g), P
+ * the planes,
  *   3D: [left, right, area, rcent] [rRL (3), mc.x] [mc.y, mc.z, dL.x, dL.y]
  *       [dL.z, dR (3)]
  *   2D: [left, right, area, rcent] [rRL (2), mc (2)] [dL (2), dR (2)]

@@ -72,12 +72,17 @@
 #define SFX_BIG_MESH (1 << 20)
 #endif
 #ifndef SFX_EGEO_U  // entries a lane of the FP32 record build forms at a time
-#define SFX_EGEO_U 4  // (3D Sedov build: 1.49 ms; 2: 1.51, 8: 1.55, one at a time: 1.69)
+#define SFX_EGEO_U 2  // (both records, 3D 1.1M / 2D 262,144 cells: 627 / 33.5 us; 4: 633 / 40.7)
 #endif
 #ifndef SFX_EGEO_U64  // the same for FP64 records
 #define SFX_EGEO_U64 4  // (3D Sedov build: 2.345 ms; 2: 2.465, one at a time: 2.455)
 #endif
-#ifndef SFX_EGEO_WAVES  // record builds over large meshes: waves per SIMD (0: all that fit)
+// Rows of a group's FP32 records that a block puts together in LDS; a group's
+// longest cell has about 23 (3D) or 10 (2D) entries, further rows go to memory
+// directly
+#define SFX_EGEO_ROWS 24
+#define SFX_EGEO_ROWS_2D 12
+#ifndef SFX_EGEO_WAVES  // FP64 record builds over large meshes: waves per SIMD (0: all that fit)
 #define SFX_EGEO_WAVES 2
 #endif
 #ifndef SFX_GATHER_KB_F64  // FP64 rows: the same registers as 8 FP32 rows
@@ -128,8 +133,8 @@ struct MeshView {
     // [ND][C] every cell's closure residual sum A r_ij/|r_ij| (mixed
     // gradients), or null where the cells' faces close
     const T* closure = nullptr;
-    // mixed pass: the faces' own values as 3 (2D) or 4 (3D) planes of F
-    // float4 (face_record_kernel), or null: read from the arrays above
+    // mixed pass: the faces' own values, 3 (2D) or 4 (3D) float4 each
+    // (face_record_kernel), or null: read from the arrays above
     const float4* frec = nullptr;
 };
 
@@ -500,20 +505,35 @@ __device__ __forceinline__ void predict_side_offset(float gamma, const double* W
 
 // ------------------------------------------------------- face records --
 
-// Planes of F float4 holding, for face f, the values the mixed face kernel
-// reads of the face itself, so that it loads them with 3 (2D) or 4 (3D)
+// F records of 3 (2D) or 4 (3D) float4 holding, for face f, the values the
+// mixed face kernel reads of the face itself, so that it loads them with 3 (2D) or 4 (3D)
 // 16-byte loads instead of 13 (2D) or 17 (3D) 4-byte ones (the kernel's
 // address unit, busy for most of its time, handles a wave's load in about
 // the same number of cycles whatever its width):
 //   3D: [left, right, area, rcent] [rRL (3), mc.x] [mc.y, mc.z, dL.x, dL.y]
 //       [dL.z, dR (3)]
 //   2D: [left, right, area, rcent] [rRL (2), mc (2)] [dL (2), dR (2)]
-// (indices as their bits).  Built once per tessellation, as the entry
+// (indices as their bits), G = 4 (3D) or 8 (2D) faces plane by plane: the
+// first float4 of faces G i to G i + G - 1, then their second ones, ... (the
+// last F % G faces among themselves).  The face kernel's loads then still fill
+// whole 64-byte pieces, and a single face, as the entry records read them,
+// lies in fewer cache lines than in planes of F (both records of 1.1M 3D
+// cells: planes 667 us, G = 2 657, 4 627, 8 661; 2D at 4 costs the face
+// kernel 2%).  Built once per tessellation, as the entry
 // records are; the values are the FP32 arrays' own, so the face fluxes are
 // bit for bit those of the array reads.
 template <int ND>
 constexpr int face_record_planes() {
     return ND == 3 ? 4 : 3;
+}
+
+// float4 index of face f's first plane; its further planes lie step apart
+template <int ND>
+__device__ __forceinline__ int64_t face_record_at(int64_t F, int64_t f, int& step) {
+    constexpr int G = ND == 3 ? 4 : 8;
+    const int64_t g0 = f & ~(int64_t)(G - 1), rest = F - g0;
+    step = rest < G ? (int)rest : G;
+    return g0 * face_record_planes<ND>() + (f - g0);
 }
 
 template <int ND>
@@ -534,9 +554,11 @@ __global__ __launch_bounds__(256) void face_record_kernel(MeshView<float> m,
         v[4 + 2 * ND + l] = m.dL[l * F + f];
         v[4 + 3 * ND + l] = m.dR[l * F + f];
     }
+    int step;
+    const int64_t at = face_record_at<ND>(F, f, step);
 #pragma unroll
     for(int q = 0; q < face_record_planes<ND>(); q++)
-        frec[q * F + f] = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+        frec[at + q * step] = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
 }
 
 // ------------------------------------------------------------- K2 grads --
@@ -554,13 +576,15 @@ template <int ND>
 __device__ __forceinline__ FaceVals<ND> load_face_record(const float4* __restrict__ frec,
                                                          int64_t F, int64_t f) {
     FaceVals<ND> o;
-    const float4 p0 = frec[f], p1 = frec[F + f], p2 = frec[2 * F + f];
+    int step;
+    const float4* r = frec + face_record_at<ND>(F, f, step);
+    const float4 p0 = r[0], p1 = r[step], p2 = r[2 * step];
     o.left = __float_as_int(p0.x);
     o.right = __float_as_int(p0.y);
     o.area = p0.z;
     o.rcent = p0.w;
     if constexpr(ND == 3) {
-        const float4 p3 = frec[3 * F + f];
+        const float4 p3 = r[3 * step];
         const float v[12] = {p1.x, p1.y, p1.z, p1.w, p2.x, p2.y, p2.z, p2.w, p3.x, p3.y, p3.z, p3.w};
 #pragma unroll
         for(int l = 0; l < ND; l++) {
@@ -770,13 +794,29 @@ __device__ __forceinline__ void load_record(const MeshView<T>& m, int64_t base, 
 // entries never matches), as that lane's entry j - off[l], written to row
 // egrp[g] + j - off[l].  A second loop writes zeros to the rows past each
 // lane's last entry.
+//
+// FP32: the rows are put together in LDS, zeros included, and written in
+// order: 32-byte pieces written one by one share their lines with other
+// entries' (both records of 1.1M 3D cells 732 us, 771 at 2 waves per SIMD;
+// staged 667).  216,000 3D cells: 81 -> 74 us, 300 MB at 4
+// TB/s.  FP64 records fill 64- or 96-byte pieces; 12 staged rows cost 3%.
+template <int ND, typename T>
+constexpr int egeo_rows() {
+    return sizeof(T) == 8 ? 0 : ND == 3 ? SFX_EGEO_ROWS : SFX_EGEO_ROWS_2D;
+}
+
 template <int ND, typename T>
 __global__ __launch_bounds__(256) void entry_geometry_grouped_kernel(MeshView<T> m,
                                                                      T* __restrict__ egeo) {
     constexpr int ER = entry_rec<ND, T>(), P = rec_planes<ND, T>();
+    constexpr int64_t RK = egeo_rows<ND, T>();
     __shared__ int64_t off[65], base[64];
+    __shared__ float4 stage[RK > 0 ? RK * P * 64 : 1];
     const int64_t g = xcd_block();
     const int64_t s0 = g * 64;
+    const int64_t r0 = m.egrp[g], K = m.egrp[g + 1] - r0;
+    const int ns = (int)((K < RK ? K : RK) * P * 64);
+    for(int t = threadIdx.x; t < ns; t += blockDim.x) stage[t] = make_float4(0.f, 0.f, 0.f, 0.f);
     const int nc = (int)((m.C - s0) < 64 ? (m.C - s0) : 64);
     if((int)threadIdx.x < 64) {
         const int l = threadIdx.x;
@@ -802,9 +842,18 @@ __global__ __launch_bounds__(256) void entry_geometry_grouped_kernel(MeshView<T>
         if(l == 0) off[0] = 0;
     }
     __syncthreads();
-    const int64_t r0 = m.egrp[g], K = m.egrp[g + 1] - r0;
     const int64_t j1 = off[nc];
     float4* out = reinterpret_cast<float4*>(egeo);
+    auto put = [&](int64_t k, int lane, const T* rec) {
+        const float4* r4 = reinterpret_cast<const float4*>(rec);
+        if(k < RK) {
+#pragma unroll
+            for(int q = 0; q < P; q++) stage[((int)k * P + q) * 64 + lane] = r4[q];
+        } else {
+#pragma unroll
+            for(int q = 0; q < P; q++) out[((r0 + k) * P + q) * 64 + lane] = r4[q];
+        }
+    };
     // the group's entry j: lane lo with off[lo] <= j < off[lo + 1], its k-th
     auto find = [&](int64_t j, int& lo_out) {
         int lo = 0, hi = nc;
@@ -848,10 +897,7 @@ __global__ __launch_bounds__(256) void entry_geometry_grouped_kernel(MeshView<T>
                     if(jb + u * (int64_t)blockDim.x >= j1) continue;
                     alignas(16) float rec[ER];
                     entry_record_from_face<ND>(fv[u], e[u], rec);
-#pragma unroll
-                    for(int q = 0; q < P; q++)
-                        out[((r0 + k[u]) * P + q) * 64 + lo[u]] =
-                                reinterpret_cast<const float4*>(rec)[q];
+                    put(k[u], lo[u], rec);
                 }
             }
             goto pad;
@@ -879,10 +925,7 @@ __global__ __launch_bounds__(256) void entry_geometry_grouped_kernel(MeshView<T>
                 if(jb + u * (int64_t)blockDim.x >= j1) continue;
                 alignas(16) double rec[ER];
                 entry_record_from_vals64<ND>(v[u], e[u], rec);
-#pragma unroll
-                for(int q = 0; q < P; q++)
-                    out[((r0 + k[u]) * P + q) * 64 + lo[u]] =
-                            reinterpret_cast<const float4*>(rec)[q];
+                put(k[u], lo[u], rec);
             }
         }
         goto pad;
@@ -892,12 +935,14 @@ __global__ __launch_bounds__(256) void entry_geometry_grouped_kernel(MeshView<T>
         const int64_t k = find(j, lo);
         alignas(16) T rec[ER];
         entry_record<ND, T>(m, m.cf_entry[base[lo] + k], rec);
-#pragma unroll
-        for(int q = 0; q < P; q++)
-            out[((r0 + k) * P + q) * 64 + lo] = reinterpret_cast<const float4*>(rec)[q];
+        put(k, lo, rec);
     }
 pad:
-    for(int64_t sl = threadIdx.x; sl < K * 64; sl += blockDim.x) {
+    if constexpr(RK > 0) {
+        __syncthreads();
+        for(int t = threadIdx.x; t < ns; t += blockDim.x) out[r0 * P * 64 + t] = stage[t];
+    }
+    for(int64_t sl = RK * 64 + threadIdx.x; sl < K * 64; sl += blockDim.x) {
         const int64_t k = sl >> 6;
         const int lane = (int)(sl & 63);
         const int64_t n = lane < nc ? off[lane + 1] - off[lane] : 0;
@@ -1854,8 +1899,8 @@ __device__ __forceinline__ void gather_cell(int64_t i, const int64_t* __restrict
 //     longer fit.  FP32 rows at 2 waves per SIMD: 526 MB read instead of 765,
 //     9% less time; FP64 rows at 1: 906 MB instead of 2,348 (2 waves: 1,325
 //     MB, 10% less time; 1 wave: 3.5% more than that);
-//   * the record build's scattered face reads: 2 waves per SIMD read 4.4 GB
-//     instead of 6.7 (FP64) and 1.7 instead of 2.9 (FP32), 8% and 3% faster.
+//   * the FP64 record build's scattered face reads: 2 waves per SIMD read 4.4
+//     GB instead of 6.7, 8% faster.
 // The gradients and the face fluxes lost time at 2 or 3 waves per SIMD and
 // moved the same bytes.  Small meshes, a few waves per SIMD in all, keep
 // their full occupancy: there the loads' latency is what counts.

@@ -26,13 +26,12 @@ hipError_t launch_entry_geometry<float>(int ndim, const flux::MeshView<float>& m
         // grouped layout: a block per group of 64 cells (the last one padded)
         if(m.C <= 0) return hipSuccess;
         const dim3 g((unsigned)((m.C + 63) / 64));  // one block per group
-        const unsigned egeo_lds = flux::occupancy_lds_bytes(SFX_EGEO_WAVES, m.C, SFX_BIG_MESH, 1024);
         if(ndim == 3)
-            hipLaunchKernelGGL((flux::entry_geometry_grouped_kernel<3, float>), g, dim3(256), egeo_lds,
-                               s, m, egeo);
+            hipLaunchKernelGGL((flux::entry_geometry_grouped_kernel<3, float>), g, dim3(256), 0, s, m,
+                               egeo);
         else
-            hipLaunchKernelGGL((flux::entry_geometry_grouped_kernel<2, float>), g, dim3(256), egeo_lds,
-                               s, m, egeo);
+            hipLaunchKernelGGL((flux::entry_geometry_grouped_kernel<2, float>), g, dim3(256), 0, s, m,
+                               egeo);
         return hipGetLastError();
     }
     if(E <= 0) return hipSuccess;

@@ -97,7 +97,7 @@ hipError_t launch_gather_fp64(int ndim, int64_t C, int64_t F, const int64_t* gof
                               const int32_t* gent, const double* dQL, double* dQ,
                               hipStream_t s);
 // flux_pass_mixed.hip: the mixed face kernel's per-face records (frec: 3 or
-// 4 planes of m.F float4, see flux::face_record_kernel)
+// 4 float4 a face, m.F faces, see flux::face_record_kernel)
 hipError_t launch_face_records(int ndim, const flux::MeshView<float>& m, float* frec,
                                hipStream_t s);
 hipError_t launch_gather_mixed(int ndim, int64_t C, int64_t F, const int64_t* goff,
