@@ -506,9 +506,9 @@ __device__ __forceinline__ void predict_side_offset(float gamma, const double* W
 // ------------------------------------------------------- face records --
 
 // F records of 3 (2D) or 4 (3D) float4 holding, for face f, the values the
-// mixed face kernel reads of the face itself, so that it loads them with 3 (2D) or 4 (3D)
-// 16-byte loads instead of 13 (2D) or 17 (3D) 4-byte ones (the kernel's
-// address unit, busy for most of its time, handles a wave's load in about
+// mixed face kernel reads of the face itself, so that it loads them with 3
+// (2D) or 4 (3D) 16-byte loads instead of 13 (2D) or 17 (3D) 4-byte ones (the
+// kernel's address unit, busy for most of its time, handles a wave's load in about
 // the same number of cycles whatever its width):
 //   3D: [left, right, area, rcent] [rRL (3), mc.x] [mc.y, mc.z, dL.x, dL.y]
 //       [dL.z, dR (3)]
@@ -1505,9 +1505,9 @@ __device__ __forceinline__ void load_grad(const T* grad, int64_t C, int64_t cell
 // The activity flag read for every cell of a mesh without an activity array.
 static __device__ const uint8_t kAllActive = 1;
 
-// ROOT: Consts::root of the exact solvers (0 for HLLC).  MIXED: 0 = FP64 parity solvers, 1 = mixed solvers (and, for a periodic
-// face whose other copy has a lower index, no evaluation: the gather applies
-// that copy's flux with the opposite sign).
+// ROOT: Consts::root of the exact solvers (0 for HLLC).  MIXED: 0 = FP64
+// parity solvers, 1 = mixed solvers (and, for a periodic face whose other copy
+// has a lower index, no evaluation: that copy writes both rows).
 // Face f: its flux goes to dQL[(f + qshift) * NC ...]; the gradients of its
 // cells are read at grad[(cell + gshift) * ND * NC ...]; the solver counters
 // are added to cnt.
