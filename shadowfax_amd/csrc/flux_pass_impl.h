@@ -1890,20 +1890,12 @@ __device__ __forceinline__ void gather_cell(int64_t i, const int64_t* __restrict
 // LDS bytes a launch over a mesh of `items` cells reserves per block of 256
 // threads (one wave per SIMD, static_lds bytes of its own), so that at most
 // `waves` blocks share a CU's 160 KB; meshes below `big` cells keep every
-// block that fits.  Some kernels here move far fewer bytes at low occupancy,
-// measured on the 3D Sedov mesh (2,097,152 cells, 16.5M faces):
-//   * the gather reads every face's row twice, from its left and its right
-//     cell; the right cell's read hits the XCD's 4 MB L2 only while the row
-//     is still there, and with every block the CU can hold in flight (8
-//     waves per SIMD: 65,536 cells an XCD) the rows between the two reads no
-//     longer fit.  FP32 rows at 2 waves per SIMD: 526 MB read instead of 765,
-//     9% less time; FP64 rows at 1: 906 MB instead of 2,348 (2 waves: 1,325
-//     MB, 10% less time; 1 wave: 3.5% more than that);
-//   * the FP64 record build's scattered face reads: 2 waves per SIMD read 4.4
-//     GB instead of 6.7, 8% faster.
-// The gradients and the face fluxes lost time at 2 or 3 waves per SIMD and
-// moved the same bytes.  Small meshes, a few waves per SIMD in all, keep
-// their full occupancy: there the loads' latency is what counts.
+// block that fits.  The FP64 record build's scattered face reads move far
+// fewer bytes so: 3D Sedov mesh (2,097,152 cells, 16.5M faces), 2 waves per
+// SIMD, 4.4 GB instead of 6.7, 8% faster.  The gradients and the face fluxes
+// lost time at 2 or 3 waves per SIMD and moved the same bytes.  Small meshes,
+// a few waves per SIMD in all, keep their full occupancy: there the loads'
+// latency is what counts.
 inline unsigned occupancy_lds_bytes(int waves, int64_t items, int64_t big, unsigned static_lds) {
     if(waves <= 0 || items < big) return 0;
     const unsigned per = ((163840u / (unsigned)waves) & ~1023u) - 1024u;

@@ -92,11 +92,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void e
     block_add_counters(ctr, cv);
 }
 
-// One lane solves one problem (see ScalarIn).
+// One lane solves one problem (see ScalarIn).  Bounds as the batch kernels':
+// the general path that they share, out of line, gets the registers of its
+// least bound caller, and they reserve as many (244 instead of 128: 262,144
+// problems 60 us instead of 47).
 template <int ND, int KIND, int ROOT, bool SOLVE>
-__global__ __launch_bounds__(64) void scalar_kernel(Consts c, ScalarIn in,
-                                                    ScalarOut* __restrict__ out,
-                                                    unsigned long long* __restrict__ ctr) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void scalar_kernel(
+        Consts c, ScalarIn in, ScalarOut* __restrict__ out, unsigned long long* __restrict__ ctr) {
     if(threadIdx.x) return;
     unsigned iters = 0, brent = 0, vac = 0;
     double f[ND + 2], mach = in.mach;
