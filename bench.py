@@ -606,10 +606,10 @@ def main():
     fp3["host_mesh_s"] = t_mesh
     ms = fp3["mixed"]["ms_mean"]
     F = b3["F"]
-    face_k = "sfx::flux::face_flux_kernel<3, 0, 1, float, double, true>"
+    face_k = "sfx::flux::face_flux_kernel<3, 0, 1, float, double, true, 5>"
     roof = roofline(b3, fp3, "3d", face_k,
                     ["sfx::flux::gradient_lds_kernel<3>", face_k,
-                     "sfx::flux::gather_kernel<3, 1, float, 16>"])
+                     "sfx::flux::gather_kernel<3, float, 48, 256, 1, 832, 4>"])
     out = {"metric": METRIC, "value": F / (ms * 1e-3), "unit": "face-fluxes/s", "n_gpus": 1,
            "steps": args.steps, "warmup": args.warmup, "ms_per_step": ms,
            "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
@@ -653,10 +653,10 @@ def main():
         fp2["host_mesh_s"] = t2
         fp2["workload"] = ("2D periodic unit box, 512x512 jittered generators (seed %d) in "
                            "Hilbert order, Kelvin-Helmholtz, HLLC" % SEED_2D)
-        face2 = "sfx::flux::face_flux_kernel<2, 1, 1, float, double, true>"
+        face2 = "sfx::flux::face_flux_kernel<2, 1, 1, float, double, true, 0>"
         fp2["roofline"] = roofline(b2, fp2, "2d", face2,
                                    ["sfx::flux::gradient_kernel<2, float, double, true>", face2,
-                                    "sfx::flux::gather_kernel<2, 1, float, 0>"])
+                                    "sfx::flux::gather_kernel<2, float, 64, 128, 2, 448, 4>"])
         measured_fracs(fp2["roofline"], mp)
         out["fluxpass_2d_kh"] = fp2
         del b2
