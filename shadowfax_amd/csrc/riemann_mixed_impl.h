@@ -634,8 +634,9 @@ __device__ uint8_t hllc_mixed(const CF& cf, const Consts& c, const double* WL, d
 // mixed 3D faces of 250,000 cells 104 -> 89 us.  The error against FP64 is
 // the FP32 output's rounding both ways (rms 2.4e-8, maximum 6e-8).
 //
-// Sides out of FP32's comfortable range, zero or non-finite states go through
-// the general iteration below (exact_general), out of line.
+// Ratios of the sides out of FP32's comfortable range, zero or non-finite
+// states go through the general iteration below (exact_general), out of line;
+// the units of density and pressure do not matter (cgs: 1e-31 g/cm^3).
 
 struct RootCase {
     double uLd, uRd, aLd, aRd;  // FP64 normal velocities and sound speeds
@@ -666,15 +667,15 @@ __device__ __forceinline__ void root_setup(const CF& c, const Consts& cd, bool r
     s.uLd = uL;
     s.uRd = uR;
     const double rL = WL[0], pL = WL[P], rR = WR[0], pR = WR[P];
-    // false for NaNs too
-    const double rmin = smin(rL, rR), rmax = smax(rL, rR), pmin = smin(pL, pR),
-                 pmax = smax(pL, pR);
-    if(!(rL >= 1e-30 && rR >= 1e-30 && pL >= 1e-30 && pR >= 1e-30 && rmin >= 1e-30 &&
-         pmin >= 1e-30 && rmax <= 1e30 && pmax <= 1e30 && pmax <= 1e18 * pmin &&
-         fabs(uL) <= 1e12 && fabs(uR) <= 1e12)) {
+    // Densities and pressures enter the FP32 iteration by their ratios only, so
+    // any unit will do; false for NaNs too
+    const double rmax = fmax(rL, rR), pmin = fmin(pL, pR), pmax = fmax(pL, pR);
+    if(!(rL >= 1e-100 && rR >= 1e-100 && pL >= 1e-100 && pR >= 1e-100 && rmax <= 1e100 &&
+         pmax <= 1e100 && pmax <= 1e18 * pmin)) {
         s.phase = EX_GENERAL;
         return;
     }
+    const double ipL = fp64::rcp64(pL);
     s.aLd = fp64::sqrt64(cd.gamma * pL * fp64::rcp64(rL));
     s.aRd = fp64::sqrt64(cd.gamma * pR * fp64::rcp64(rR));
     const double dud = uR - uL, taLd = cd.tdgm1 * s.aLd, taRd = cd.tdgm1 * s.aRd;
@@ -684,21 +685,25 @@ __device__ __forceinline__ void root_setup(const CF& c, const Consts& cd, bool r
     }
     s.phase = EX_ITER;
     s.pure_newton = dud - (taLd + taRd) < cd.cutoff;
-    const float pLf = (float)pL, pRf = (float)pR, aL = (float)s.aLd, aR = (float)s.aRd;
+    const float aL = (float)s.aLd, aR = (float)s.aRd;
     const float du = (float)dud, taL = (float)taLd, taR = (float)taRd;
-    if(!(fmaxf(aL, aR) <= 1e8f * fminf(aL, aR) && -du <= 1e10f * fmaxf(aL, aR))) {
+    // the ram pressure: p* is at most 2 (pmax + ram), 4e24 pmin
+    const double ram = rmax * dud * dud;
+    const float amin = fminf(aL, aR), amax = fmaxf(aL, aR);
+    if(!(ram <= 1e24 * pmin && amax <= 1e8f * amin && amin >= 1e-25f && amax <= 1e20f)) {
         s.phase = EX_GENERAL;
         return;
     }
     s.du = du;
     s.taL = taL;
     s.taR = taR;
-    const float rpL = rcpf(pLf);
-    s.q = exp2f_fast(cd.rootf * log2f_fast(pLf * rcpf(pRf)));
     // initial guess, ExactRiemannSolver.cpp:644-673, in units of pL
-    const float x = pRf * rpL, xsum = 1.f + x, xmin = fminf(1.f, x), xmax = fmaxf(1.f, x);
+    const float x = (float)(pR * ipL), rx = rcpf(x);
+    s.q = exp2f_fast(-cd.rootf * log2f_fast(x));
+    const float xsum = 1.f + x, xmin = fminf(1.f, x), xmax = fmaxf(1.f, x);
     const float xfloor = c.halftol * xsum;
-    const float xpv = fmaxf(xfloor, 0.5f * xsum - 0.125f * du * (float)(rL + rR) * (aL + aR) * rpL);
+    const float xpv = fmaxf(xfloor, 0.5f * xsum -
+                                            (float)(0.125 * dud * (rL + rR) * (s.aLd + s.aRd) * ipL));
     float xg;
     if(xmax <= 2.f * xmin && xmin <= xpv && xpv <= xmax) {
         xg = xpv;
@@ -707,8 +712,9 @@ __device__ __forceinline__ void root_setup(const CF& c, const Consts& cd, bool r
     } else {
         const float k = (float)cd.kshock;
         const float gL = k * aL * __builtin_amdgcn_rsqf(xpv + c.gm1dgp1),
-                    gR = k * aR * __builtin_amdgcn_rsqf(xpv * rcpf(x) + c.gm1dgp1);
-        xg = (gL + gR - du) * rcpf(gL + gR * rcpf(x));
+                    gR = k * aR * __builtin_amdgcn_rsqf(xpv * rx + c.gm1dgp1);
+        // (far from the truth where a light side meets a heavy one)
+        xg = fminf((gL + gR - du) * rcpf(gL + gR * rx), (float)(2.0 * (pmax + ram) * ipL));
     }
     s.z = exp2f_fast(cd.rootf * log2f_fast(fmaxf(xfloor, xg)));
 }
@@ -744,9 +750,12 @@ __device__ __forceinline__ void root_iterate(const CF& c, const Consts& cd, Root
             phase = EX_STUCK;
             break;
         }
-        const float zn = fmaxf(z - z * f * rcpf(d), 1e-7f * z);
-        const bool done = fabsf(zn - z) <= (SFX_MIXED_STEP_TOL / ROOT) * (zn + z);
-        z = zn;
+        // zn = z (1 - t) within z 1e-7 and 8 z: from left of the root one step
+        // may overshoot it by any factor, and 8 a step keep both sides' powers
+        // below FP32's end
+        const float t = __builtin_amdgcn_fmed3f(f * rcpf(d), -7.f, 0.9999999f);
+        const bool done = fabsf(t) <= (SFX_MIXED_STEP_TOL / ROOT) * (2.f - t);
+        z -= z * t;
         if(done) {
             phase = EX_DONE;
             break;

@@ -62,3 +62,71 @@ def test_mixed_exact_over_its_range(device, gamma, nd):
                            ((0, 1000), (1000, 2000), (2000, 3000), (3000, 4000), (4000, 5500),
                             (5500, 7000))], flush=True)
     assert err.max() <= TOL
+
+
+def limit_blocks(nd, seed):
+    """The ends of what the iteration takes: densities and pressures in units
+    from 1e-31 (gas in cgs) to 1e30 and beyond FP32's range, streams that
+    collide up to a ram pressure of 1e23 times the lower pressure (the limit
+    is 1e24), a light hot side against a heavy cold one (sound speeds
+    1e8, pressures 1e15 apart), and speeds from 1e-21 to 1e16.  Sides that collide differ in density: two
+    equal ones leave the contact at rest but for round-off of their speeds,
+    1e-16 times 1e10 sound speeds in any precision."""
+    b = WK.riemann_batch(6000, seed=seed, family="uniform", ndim=nd, round32=False)
+    WL, WR, n = b["WL"], b["WR"], b["n"]
+    r = np.random.RandomState(seed)
+    u, k = r.uniform(size=6000), np.arange(6000)
+
+    def scale(m, s):
+        for W in (WL, WR):
+            W[0, m] *= s
+            W[-1, m] *= s
+
+    def collide(m, lo):
+        # the closing speed from the lower sound speed (lo = 0) to the limit
+        a = np.sqrt(np.minimum(WL[-1, m] / WL[0, m], WR[-1, m] / WR[0, m]))
+        top = np.sqrt(1e23 * np.minimum(WL[-1, m], WR[-1, m]) / np.maximum(WL[0, m], WR[0, m]))
+        s = a * (top / a) ** r.uniform(lo, 1, m.sum())
+        WL[1:1 + nd, m] += 0.5 * s * n[:, m]
+        WR[1:1 + nd, m] -= 0.5 * s * n[:, m]
+
+    scale(k < 1000, 1e-31)
+    m = (k >= 1000) & (k < 2000)
+    scale(m, 10.0 ** (180 * u[m] - 90))
+    m = (k >= 2000) & (k < 3000)  # densities and pressures about 1e30
+    WL[0, m] = WL[-1, m] = WR[-1, m] = 10.0 ** (29 + u[m])
+    WR[0, m] = WL[0, m] * r.uniform(2, 8, m.sum())
+    collide(m, 0.7)
+    m = (k >= 3000) & (k < 4000)
+    scale(m, 10.0 ** (40 * u[m] - 20))
+    collide(m, 0)
+    m = (k >= 4000) & (k < 5000)  # heavy and cold left, light and hot right
+    WR[-1, m] = WL[-1, m] * 10.0 ** (15 * u[m])
+    WR[0, m] = WL[0, m] * (WR[-1, m] / WL[-1, m]) * 10.0 ** -(16 * r.uniform(size=m.sum()))
+    collide(m, 0)
+    m = k >= 5000  # speeds in other units
+    s = 10.0 ** (37 * u[m] - 21)
+    for W in (WL, WR):
+        W[1:1 + nd, m] *= s
+        W[-1, m] *= s * s
+    return WL, WR, n
+
+
+@pytest.mark.parametrize("nd", [2, 3])
+@pytest.mark.parametrize("gamma", [5.0 / 3.0, 1.4])
+def test_mixed_exact_units_and_limits(device, gamma, nd):
+    import torch
+    print("case", gamma, nd, flush=True)
+    WL, WR, n = limit_blocks(nd, 29)
+    t = lambda a: torch.tensor(np.ascontiguousarray(a), device=device)
+    out = {}
+    for prec in ("fp64", "mixed"):
+        s = RiemannSolver(0, nd, gamma, 1e-8, -5.0, prec)
+        st = torch.zeros(WL.shape[1], dtype=torch.uint8, device=device)
+        F = s.solve_for_flux_batch(t(WL), t(WR), t(n), status=st)
+        torch.cuda.synchronize()
+        out[prec] = (F.cpu().numpy(), st.cpu().numpy())
+    assert not out["fp64"][1].any() and not out["mixed"][1].any()
+    err = normwise_error(out["mixed"][0], out["fp64"][0], WL, WR, gamma)
+    print("max by block", [float(err[a:a + 1000].max()) for a in range(0, 6000, 1000)], flush=True)
+    assert err.max() <= TOL
