@@ -673,6 +673,17 @@ __device__ __forceinline__ void root_setup(const CF& c, const Consts& cd, bool r
     if(!(rL >= 1e-100 && rR >= 1e-100 && pL >= 1e-100 && pR >= 1e-100 && rmax <= 1e100 &&
          pmax <= 1e100 && pmax <= 1e18 * pmin)) {
         s.phase = EX_GENERAL;
+        // vacuum beside such a gas, or on both sides: closed forms here (out of
+        // line 1,048,576 problems took 169 us, 16 here)
+        const bool eL = !(rL != 0.0), eR = !(rR != 0.0);
+        const auto gas = [](double r, double p) {
+            return r >= 1e-100 && r <= 1e100 && p >= 1e-100 && p <= 1e100;
+        };
+        if((eL || eR) && (eL || gas(rL, pL)) && (eR || gas(rR, pR))) {
+            s.phase = EX_VACUUM;
+            s.aLd = eL ? 0.0 : fp64::sqrt64(cd.gamma * pL * fp64::rcp64(rL));
+            s.aRd = eR ? 0.0 : fp64::sqrt64(cd.gamma * pR * fp64::rcp64(rR));
+        }
         return;
     }
     const double ipL = fp64::rcp64(pL);
