@@ -90,6 +90,12 @@ __attribute__((amdgpu_waves_per_eu(ROOT != 0 ? SFX_MIXED_WAVES : 1, 10))) void s
 // prefix sum of their counts, resumes each problem where it stopped and
 // finishes it.  The iteration sequence per problem is unchanged, so results
 // are bit-identical to the one-kernel path.
+//
+// Problems of the general iteration are queued as they are (it = -1) and
+// solved at the end of phase 2: phase 1 holds no call.  With one, phase 1
+// spilled 76 registers at the 6 waves of the one-kernel path, and 4,194,304
+// 3D problems queued after 4 iterations took 240 us, 128 so (phase 2 at 4
+// waves, where neither kernel spills).
 
 struct Straggler {
     int32_t i;
@@ -97,7 +103,8 @@ struct Straggler {
     int32_t it;
 };
 
-// the two iterations' parts under one name
+// the two iterations' parts under one name; finish takes no problem of phase
+// EX_GENERAL
 template <int ND, int ROOT>
 struct Parts {
     using Case = std::conditional_t<ROOT != 0, RootCase, ExactCase>;
@@ -130,7 +137,7 @@ struct Parts {
                                                      const double* n, const double* v, bool refl,
                                                      double* F, unsigned& iters, unsigned& vac) {
         if constexpr(ROOT != 0)
-            return root_finish<ND, ROOT>(c, cd, s, WL, WR, n, v, refl, F, iters, vac);
+            return root_finish<ND, ROOT, false>(c, cd, s, WL, WR, n, v, refl, F, iters, vac);
         else
             return exact_finish<ND>(c, cd, s, WL, WR, n, v, F, iters, vac);
     }
@@ -154,7 +161,6 @@ struct Parts {
             s.hi = g.hi;
         }
         s.it = g.it;
-        s.phase = EX_ITER;
     }
 };
 
@@ -203,7 +209,7 @@ __attribute__((amdgpu_waves_per_eu(ROOT != 0 ? SFX_MIXED_WAVES : 1, 10))) void e
         X::setup(c, cd, r, wl64, wr64, n64, s);
         if(s.phase == EX_ITER) X::iterate(c, cd, s, stop);
     }
-    const bool strag = valid && s.phase == EX_ITER;
+    const bool strag = valid && (s.phase == EX_ITER || s.phase == EX_GENERAL);
     // slots in the block's segment: a ballot per wave, one LDS atomic per wave
     const unsigned long long mask = __ballot(strag);
     const int lane = __lane_id();
@@ -214,7 +220,12 @@ __attribute__((amdgpu_waves_per_eu(ROOT != 0 ? SFX_MIXED_WAVES : 1, 10))) void e
         const unsigned slot = base + (unsigned)__popcll(mask & ((1ull << lane) - 1ull));
         Straggler g;
         g.i = (int32_t)i;
-        X::save(s, g);
+        if(s.phase == EX_GENERAL) {
+            g.p = g.lo = g.hi = 0.f;
+            g.it = -1;
+        } else {
+            X::save(s, g);
+        }
         queue[(int64_t)blockIdx.x * blockDim.x + slot] = g;
     } else if(valid) {
         double f[NC];
@@ -233,7 +244,7 @@ __attribute__((amdgpu_waves_per_eu(ROOT != 0 ? SFX_MIXED_WAVES : 1, 10))) void e
 
 template <int ND, typename T, int ROOT>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(ROOT != 0 ? SFX_MIXED_WAVES : 1, 10))) void exact_phase2_kernel(
+__attribute__((amdgpu_waves_per_eu(ROOT != 0 ? 4 : 1, 10))) void exact_phase2_kernel(
         CF c, Consts cd, int64_t N, const T* __restrict__ WL, const T* __restrict__ WR,
         const T* __restrict__ n, const T* __restrict__ v, const uint8_t* __restrict__ refl,
         T* __restrict__ F, uint8_t* __restrict__ status, unsigned long long* __restrict__ ctr,
@@ -254,11 +265,26 @@ __attribute__((amdgpu_waves_per_eu(ROOT != 0 ? SFX_MIXED_WAVES : 1, 10))) void e
     __syncthreads();
     const unsigned total = s_pre[kSegs];
     unsigned iters = 0, vac = 0, fail = 0, done = 0;
-    for(unsigned k = threadIdx.x; k < total; k += blockDim.x) {
+    int general = 0;
+    const auto entry = [&](unsigned k) {
         int q = 0;
         while(q + 1 < kSegs && s_pre[q + 1] <= k) q++;
-        const Straggler g = queue[(seg0 + q) * blockDim.x + (k - s_pre[q])];
+        return queue[(seg0 + q) * blockDim.x + (k - s_pre[q])];
+    };
+    const auto put = [&](int64_t i, uint8_t st, const double* f) {
+#pragma unroll
+        for(int r = 0; r < NC; r++) F[r * N + i] = (T)f[r];
+        if(status) status[i] = st;
+        fail += st != 0;
+        done++;
+    };
+    for(unsigned k = threadIdx.x; k < total; k += blockDim.x) {
+        const Straggler g = entry(k);
         const int64_t i = g.i;
+        if(ROOT != 0 && g.it < 0) {
+            general = 1;
+            continue;
+        }
         double wl64[NC], wr64[NC], n64[ND], v64[ND], f[NC];
         load_problem<ND, T>(N, i, WL, WR, n, v, wl64, wr64, n64, v64);
         const bool rf = refl ? refl[i] != 0 : false;
@@ -266,12 +292,24 @@ __attribute__((amdgpu_waves_per_eu(ROOT != 0 ? SFX_MIXED_WAVES : 1, 10))) void e
         X::setup(c, cd, rf, wl64, wr64, n64, s);
         X::restore(g, s);
         X::iterate(c, cd, s, c.itmax);
-        const uint8_t st = X::finish(c, cd, s, wl64, wr64, n64, v64, rf, f, iters, vac);
-#pragma unroll
-        for(int r = 0; r < NC; r++) F[r * N + i] = (T)f[r];
-        if(status) status[i] = st;
-        fail += st != 0;
-        done++;
+        put(i, X::finish(c, cd, s, wl64, wr64, n64, v64, rf, f, iters, vac), f);
+    }
+    // the general iteration's problems in a loop of their own: a call in the
+    // one above would spill its values
+    if constexpr(ROOT != 0) {
+        if(__syncthreads_or(general))
+            for(unsigned k = threadIdx.x; k < total; k += blockDim.x) {
+                const Straggler g = entry(k);
+                if(g.it >= 0) continue;
+                double wl64[NC], wr64[NC], n64[ND], v64[ND], f[NC];
+                load_problem<ND, T>(N, g.i, WL, WR, n, v, wl64, wr64, n64, v64);
+                unsigned vk = 0;
+                put(g.i,
+                    call_general<ND, 1>(c, cd, wl64, wr64, n64, v64, refl ? refl[g.i] != 0 : false,
+                                        f, iters, vk),
+                    f);
+                vac += vk;
+            }
     }
     const unsigned cv[CNT_N] = {done, 0u, vac, iters, fail};
     block_add_counters(ctr, cv);

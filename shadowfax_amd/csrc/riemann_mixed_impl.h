@@ -794,14 +794,15 @@ __device__ __forceinline__ void root_side_d(const Consts& cd, double a, double r
     }
 }
 
-// the general iteration out of line, on the same inputs
+// the general iteration out of line, on the same inputs; a copy per SITE, since
+// the callers of one copy reserve the registers of the least bound of them
 template <int ND>
 struct MixedGeneral {
     double WL[ND + 2], WR[ND + 2], n[ND], v[ND], F[ND + 2];
     unsigned iters, vac;
     bool reflective;
 };
-template <int ND>
+template <int ND, int SITE>
 __device__ __attribute__((noinline)) uint8_t exact_general(CF c, Consts cd, MixedGeneral<ND>* g) {
     constexpr int NC = ND + 2;
     float wl[NC], wr[NC], nn[ND];
@@ -818,35 +819,45 @@ __device__ __attribute__((noinline)) uint8_t exact_general(CF c, Consts cd, Mixe
     return exact_finish<ND>(c, cd, s, g->WL, g->WR, g->n, g->v, g->F, g->iters, g->vac);
 }
 
-template <int ND, int ROOT>
+template <int ND, int SITE>
+__device__ __forceinline__ uint8_t call_general(const CF& c, const Consts& cd, const double* WL,
+                                                const double* WR, const double* n,
+                                                const double* v, bool reflective, double* F,
+                                                unsigned& iters, unsigned& vac) {
+    constexpr int NC = ND + 2;
+    MixedGeneral<ND> g;
+#pragma unroll
+    for(int k = 0; k < NC; k++) {
+        g.WL[k] = WL[k];
+        g.WR[k] = WR[k];
+    }
+#pragma unroll
+    for(int d = 0; d < ND; d++) {
+        g.n[d] = n[d];
+        g.v[d] = v[d];
+    }
+    g.iters = iters;
+    g.vac = vac;
+    g.reflective = reflective;
+    const uint8_t st = exact_general<ND, SITE>(c, cd, &g);
+#pragma unroll
+    for(int k = 0; k < NC; k++) F[k] = g.F[k];
+    iters = g.iters;
+    vac = g.vac;
+    return st;
+}
+
+// GENERAL: problems of phase EX_GENERAL may come
+template <int ND, int ROOT, bool GENERAL = true>
 __device__ __forceinline__ uint8_t root_finish(const CF& c, const Consts& cd, const RootCase& s,
                                                const double* WL, const double* WR,
                                                const double* n, const double* v,
                                                bool reflective, double* F, unsigned& iters,
                                                unsigned& vac) {
     constexpr int NC = ND + 2, P = ND + 1;
-    if(s.phase == EX_GENERAL) {
-        MixedGeneral<ND> g;
-#pragma unroll
-        for(int k = 0; k < NC; k++) {
-            g.WL[k] = WL[k];
-            g.WR[k] = WR[k];
-        }
-#pragma unroll
-        for(int d = 0; d < ND; d++) {
-            g.n[d] = n[d];
-            g.v[d] = v[d];
-        }
-        g.iters = iters;
-        g.vac = vac;
-        g.reflective = reflective;
-        const uint8_t st = exact_general<ND>(c, cd, &g);
-#pragma unroll
-        for(int k = 0; k < NC; k++) F[k] = g.F[k];
-        iters = g.iters;
-        vac = g.vac;
-        return st;
-    }
+    if constexpr(GENERAL)
+        if(s.phase == EX_GENERAL)
+            return call_general<ND, 0>(c, cd, WL, WR, n, v, reflective, F, iters, vac);
     double sol[NC];
     if(s.phase == EX_VACUUM) {
         vac = 1;

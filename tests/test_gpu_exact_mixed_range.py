@@ -130,3 +130,31 @@ def test_mixed_exact_units_and_limits(device, gamma, nd):
     err = normwise_error(out["mixed"][0], out["fp64"][0], WL, WR, gamma)
     print("max by block", [float(err[a:a + 1000].max()) for a in range(0, 6000, 1000)], flush=True)
     assert err.max() <= TOL
+
+
+@pytest.mark.parametrize("nd", [2, 3])
+@pytest.mark.parametrize("gamma", [5.0 / 3.0, 1.4, 1.66667])
+def test_split_equals_one_kernel_over_the_range(device, gamma, nd):
+    """The two-phase solve on problems of every path: the iteration in the
+    n-th root, the general one beyond its range (pressure ratios of 1e20, no
+    pressure, NaN), vacuum.  The same bits, status and counters."""
+    import torch
+    print("case", gamma, nd, flush=True)
+    WL, WR, n = blocks(nd, 37)
+    WR[-1, 100:160] = 1e-20 * WL[-1, 100:160]
+    WR[-1, 300:310] = 0.0
+    WL[0, 800:803] = np.nan
+    WL[:, 1700:1740] = 0.0
+    WR[-1, 5600:5700:3] *= 1e-25
+    t = lambda a: torch.tensor(np.ascontiguousarray(a), device=device)
+    out = []
+    for split in (0, 1, 3):
+        s = RiemannSolver(0, nd, gamma, 1e-8, -5.0, "mixed")
+        s.set_split(split)
+        st = torch.zeros(WL.shape[1], dtype=torch.uint8, device=device)
+        F = s.solve_for_flux_batch(t(WL), t(WR), t(n), status=st)
+        torch.cuda.synchronize()
+        out.append((F.cpu().numpy(), st.cpu().numpy(), s.stats()))
+    for F, st, c in out[1:]:
+        assert np.array_equal(F, out[0][0], equal_nan=True)
+        assert np.array_equal(st, out[0][1]) and c == out[0][2]
