@@ -440,12 +440,13 @@ __device__ uint8_t ex_solve_steps(const Consts& c, const double* WL, const doubl
 //
 // The reference's iteration -- guess, Newton steps, Brent's method over
 // [0, guess] from a guess right of the root -- with the same tests, so that
-// it ends at the same iterate (Brent's method stops up to 1e-8 from the
-// root: in 1 of 20,000 problems its flux is more than 1e-12 from the root's),
-// over a pressure function that costs a third.  With n = 2 gamma/(gamma-1)
-// and in units of a side's own pressure, x = p/pK,
-//   shock:        f = aK k (x - 1)/sqrt(x + (g-1)/(g+1)),  k^2 = 2/(g (g+1))
-//   rarefaction:  f = 2 aK/(g-1) (y - 1),  y = x^(1/n),  x f' = aK/g y
+// but for the round-off of the guess, the steps and the pressure function it
+// ends at the same iterate (Brent's method stops up to 1e-8 from the root: in
+// 1 of 20,000 problems its flux is more than 1e-12 from the root's), over a
+// pressure function that costs a third.  With n = 2 gamma/(gamma-1) and x =
+// p/pK,
+//   shock:        f = (p - pK) sA/sqrt(p + (g-1)/(g+1) pK),  sA^2 = 2/((g+1) rhoK)
+//   rarefaction:  f = 2 aK/(g-1) (y - 1),  y = x^(1/n),  p f' = aK/g y
 // one inverse square root or one n-th root a side and step, values and
 // derivative together, where pow() was called for each (226 instructions a
 // call).  A guess whose f is round-off
@@ -458,9 +459,11 @@ __device__ uint8_t ex_solve_steps(const Consts& c, const double* WL, const doubl
 // 262,144 problems of log-uniform states 280 -> 48 us (their 38 MB need 7),
 // 4,194,304 with vacuum and shocks 3264 -> 480 us, 1,000 problems 157 -> 26 us;
 // 4 waves per SIMD (128 VGPRs; the general path alone would take 244).
-// Normwise error against long double, 80,000 problems: rms 1.74e-14 (gamma
-// 5/3) and 5.7e-15 (7/5), maximum 3.4e-12 and 1.0e-12 both ways -- Brent's
-// stopping error -- and median 1.0e-16 both ways.
+// Error of the fluxes against 80-bit arithmetic, in units of a problem's
+// largest, 60,000 log-uniform 3D problems, step by step -> here: median 3.9e-16
+// -> 2.9e-16 (gamma 5/3), 2.9e-16 -> 2.2e-16 (7/5), 2.7e-16 both (1.66667); of
+// states a few percent apart 2.4e-16 -> 1.9e-16; the largest (2e-11 to 5e-11)
+// are Brent's stopping error both ways.
 //
 // Problems with a zero, negative, non-finite or extreme density or pressure
 // go through ex_solve_steps, whose comparisons decide as the reference's do on
@@ -471,18 +474,24 @@ __device__ uint8_t ex_solve_steps(const Consts& c, const double* WL, const doubl
 // x^(1/n) for x in FP32 range and rx = 1/x to 2^-40 or better: from the FP32
 // estimate y0 (relative error below 4e-6) by the series of (1 - d)^(-1/n),
 // d = 1 - y0^n/x, whose third term is below round-off; rootk carries what the
-// rounded gamma's exponent differs from 1/n by
+// rounded gamma's exponent differs from 1/n by.  ym1: the root less 1, without
+// the rounding of the root (a rarefaction's share of the pressure function is
+// that difference, small where two states are alike).
 template <int ROOT>
-__device__ __forceinline__ double root_n(const Consts& c, double x, double rx) {
+__device__ __forceinline__ double root_n(const Consts& c, double x, double rx, double& ym1) {
     if constexpr(ROOT != 0) {
         const float lf = __builtin_amdgcn_logf((float)x);
         const double y = (double)__builtin_amdgcn_exp2f(c.rootf * lf);
         const double y2 = y * y;
         const double d = fma(-(y2 * y2), ROOT == 7 ? y2 * y : y, x) * rx;
-        return fma(y, fma(d, fma(d, c.rn2, c.rn), (double)(c.rootk * lf)), y);
+        const double e = fma(d, fma(d, c.rn2, c.rn), (double)(c.rootk * lf));
+        ym1 = fma(y, e, y - 1.0);
+        return fma(y, e, y);
     }
     (void)rx;
-    return pow(x, c.gm1d2g);
+    const double y = pow(x, c.gm1d2g);
+    ym1 = y - 1.0;
+    return y;
 }
 // a b + the rounding error of a b, into lo
 __device__ __forceinline__ double mul_err(double a, double b, double& lo) {
@@ -491,20 +500,23 @@ __device__ __forceinline__ double mul_err(double a, double b, double& lo) {
     return h;
 }
 // b^(2/(g-1)) and b^(2g/(g-1)), b >= 0; products with their rounding errors
-// carried along (plain ones would lose the digits that pow() keeps)
+// carried along (plain ones would lose the digits that pow() keeps), and fank
+// for what the gamma in use puts between n - 2 and 2/(g-1): 1.1e-15 for the
+// double 1.4, up to 1e-11 for those that count as 7/5
 template <int ROOT>
 __device__ __forceinline__ void fan_powers(const Consts& c, double b, double& r, double& p) {
     if constexpr(ROOT != 0) {
         double e2, e3, e5, e7;
+        const double k = (double)(c.fank * __builtin_amdgcn_logf((float)fmax(b, 1e-30)));
         const double b2 = mul_err(b, b, e2), b3 = mul_err(b2, b, e3), l3 = fma(e2, b, e3);
         const double b5 = mul_err(b3, b2, e5), l5 = fma(l3, b2, fma(b3, e2, e5));
         if(ROOT == 5) {
-            r = b3 + l3;
-            p = b5 + l5;
+            r = b3 + fma(b3, k, l3);
+            p = b5 + fma(b5, k, l5);
         } else {
             const double b7 = mul_err(b5, b2, e7);
-            r = b5 + l5;
-            p = b7 + fma(l5, b2, fma(b5, e2, e7));
+            r = b5 + fma(b5, k, l5);
+            p = b7 + fma(b7, k, fma(l5, b2, fma(b5, e2, e7)));
         }
     } else {
         r = pow(b, c.tdgm1);
@@ -513,25 +525,27 @@ __device__ __forceinline__ void fan_powers(const Consts& c, double b, double& r,
 }
 
 struct ExSide {
-    double p, rp, ta, ak, ag;  // pK, 1/pK, 2 aK/(g-1), k aK, aK/g
+    double p, rp, ta, sa, ag;  // pK, 1/pK, 2 aK/(g-1), sqrt(2/((g+1) rhoK)), aK/g
 };
-__device__ __forceinline__ ExSide ex_side(const Consts& c, double p, double rp, double a) {
-    return {p, rp, c.tdgm1 * a, c.kshock * a, c.ginv * a};
+__device__ __forceinline__ ExSide ex_side(const Consts& c, double p, double rp, double a,
+                                          double sa) {
+    return {p, rp, c.tdgm1 * a, sa, c.ginv * a};
 }
 // value, p times the derivative, and y (rarefaction)
 template <int ROOT>
 __device__ __forceinline__ void ex_side_f(const Consts& c, const ExSide& s, double p, double& f,
                                           double& pdf, double& y) {
-    const double x = div_by(p, s.p, s.rp);
     if(p > s.p) {
-        const double r = rsq64(x + c.gm1dgp1), xm = div_by(p - s.p, s.p, s.rp), ar = s.ak * r;
-        f = xm * ar;
-        pdf = x * ar * fma(-0.5 * xm, r * r, 1.0);
+        const double r = rsq64(fma(c.gm1dgp1, s.p, p)), d = p - s.p, ar = s.sa * r;
+        f = d * ar;
+        pdf = p * ar * fma(-0.5 * d, r * r, 1.0);
     } else {
+        const double x = div_by(p, s.p, s.rp);
         double rx = __builtin_amdgcn_rcp(x);
         rx = fma(fma(-x, rx, 1.0), rx, rx);
-        y = root_n<ROOT>(c, x, rx);
-        f = s.ta * (y - 1.0);
+        double ym1;
+        y = root_n<ROOT>(c, x, rx, ym1);
+        f = s.ta * ym1;
         pdf = s.ag * y;
     }
 }
@@ -539,11 +553,13 @@ __device__ __forceinline__ void ex_side_f(const Consts& c, const ExSide& s, doub
 // the value alone
 template <int ROOT>
 __device__ __forceinline__ double ex_side_v(const Consts& c, const ExSide& s, double p) {
+    if(p > s.p) return (p - s.p) * (s.sa * rsq64(fma(c.gm1dgp1, s.p, p)));
     const double x = div_by(p, s.p, s.rp);
-    if(p > s.p) return div_by(p - s.p, s.p, s.rp) * (s.ak * rsq64(x + c.gm1dgp1));
     double rx = __builtin_amdgcn_rcp(x);
     rx = fma(fma(-x, rx, 1.0), rx, rx);
-    return s.ta * (root_n<ROOT>(c, x, rx) - 1.0);
+    double ym1;
+    root_n<ROOT>(c, x, rx, ym1);
+    return s.ta * ym1;
 }
 
 // BrentsMethodSolve over [0, b], f(0) = fa < 0 < fb = f(b) (ExactRiemann-
@@ -615,13 +631,16 @@ __device__ __forceinline__ bool ex_brent_root(const Consts& c, const ExSide& lo,
 // a rarefaction fan, in the star region; or vacuum
 enum : int { EX_OUT = 0, EX_SHOCK = 1, EX_FAN = 2, EX_STAR = 3, EX_ZERO = 4 };
 
-// ex_solve_steps out of line: its registers and code are not the others'
+// ex_solve_steps out of line: its registers and code are not the others'.  A
+// copy each for the kernels with a root and without, which are bound to
+// different numbers of waves: callers reserve the registers of the copy's least
+// bound one.
 template <int ND>
 struct ExGeneral {
     double WL[ND + 2], WR[ND + 2], n[ND], vL, vR, sol[ND + 2], mach;
     unsigned iters, brent, vac;
 };
-template <int ND>
+template <int ND, bool HAS_ROOT>
 __device__ __attribute__((noinline)) uint8_t ex_solve_general(Consts c, ExGeneral<ND>* g) {
     return ex_solve_steps<ND>(c, g->WL, g->WR, g->n, g->vL, g->vR, g->sol, &g->mach, g->iters,
                               g->brent, g->vac);
@@ -687,8 +706,9 @@ __device__ __forceinline__ uint8_t ex_solve(const Consts& c, const double* WL, d
         }
     }
     if(!general && !vc) {
-        aL = sqrt64(div64(c.gamma * pL, rL));
-        aR = sqrt64(div64(c.gamma * pR, rR));
+        const double irL = rcp64(rL), irR = rcp64(rR);
+        aL = sqrt64(div_by(c.gamma * pL, rL, irL));
+        aR = sqrt64(div_by(c.gamma * pR, rR, irR));
         rpL = rcp64(pL);
         rpR = rcp64(pR);
         const double dv = vR - vL;
@@ -708,8 +728,9 @@ __device__ __forceinline__ uint8_t ex_solve(const Consts& c, const double* WL, d
             // one a rarefaction in most problems that take several steps, so
             // a wave's lanes run the same halves of ex_side_f
             const bool swap = pL > pR;
-            const ExSide lo = ex_side(c, pmin, swap ? rpR : rpL, swap ? aR : aL);
-            const ExSide hi = ex_side(c, pmax, swap ? rpL : rpR, swap ? aL : aR);
+            const double saL = sqrt64(div_by(c.tdgp1, rL, irL)), saR = sqrt64(div_by(c.tdgp1, rR, irR));
+            const ExSide lo = ex_side(c, pmin, swap ? rpR : rpL, swap ? aR : aL, swap ? saR : saL);
+            const ExSide hi = ex_side(c, pmax, swap ? rpL : rpR, swap ? aL : aR, swap ? saL : saR);
             // initial guess, ExactRiemannSolver.cpp:644-673
             const double psum = pL + pR, pfloor = c.tol * 0.5 * psum;
             const double ppv = smax(pfloor, 0.5 * psum - 0.125 * dv * (rL + rR) * (aL + aR));
@@ -721,15 +742,16 @@ __device__ __forceinline__ uint8_t ex_solve(const Consts& c, const double* WL, d
                 const double x = div_by(pmin, hi.p, hi.rp);
                 double rx = __builtin_amdgcn_rcp(x);
                 rx = fma(fma(-x, rx, 1.0), rx, rx);
-                const double q = root_n<ROOT>(c, x, rx);
+                double qm1;
+                const double q = root_n<ROOT>(c, x, rx, qm1);
                 const double w = div64(lo.ta + hi.ta - dv, hi.ta * q + lo.ta);
                 double wr, wp;
                 fan_powers<ROOT>(c, w, wr, wp);
                 pg = pmin * wp;
             } else {
-                const double gl = lo.ak * __builtin_amdgcn_rsq(fma(ppv, lo.rp, c.gm1dgp1)),
-                             gh = hi.ak * __builtin_amdgcn_rsq(fma(ppv, hi.rp, c.gm1dgp1));
-                pg = (gl + gh - dv) * __builtin_amdgcn_rcp(gl * lo.rp + gh * hi.rp);
+                const double gl = lo.sa * rsq64(fma(c.gm1dgp1, lo.p, ppv)),
+                             gh = hi.sa * rsq64(fma(c.gm1dgp1, hi.p, ppv));
+                pg = div64(fma(gl, lo.p, fma(gh, hi.p, -dv)), gl + gh);
             }
             pg = smax(pfloor, pg);
             double flo, fhi, dlo, dhi, ylo = 1.0, yhi = 1.0;
@@ -796,7 +818,7 @@ __device__ __forceinline__ uint8_t ex_solve(const Consts& c, const double* WL, d
         g.iters = iters;
         g.brent = brent;
         g.vac = vac;
-        st = ex_solve_general<ND>(c, &g);
+        st = ex_solve_general<ND, ROOT != 0>(c, &g);
 #pragma unroll
         for(int k = 0; k < NC; k++) sol[k] = g.sol[k];
         if(mach) *mach = g.mach;
@@ -838,11 +860,9 @@ __device__ __forceinline__ uint8_t ex_solve(const Consts& c, const double* WL, d
         if(mode == EX_SHOCK) {
             sol[0] = div64(rK * (x + c.gm1dgp1), fma(c.gm1dgp1, x, 1.0));
         } else {
-            // x^(1/g) = x/y^2 = y^(n-2) (n = 7: y^5 would carry 5 times y's error)
-            const double y2 = y * y;
-            sol[0] = ROOT == 5   ? rK * (y2 * y)
-                     : ROOT == 7 ? (y > 0. ? div64(rK * x, y2) : 0.)
-                                 : rK * pow(x, c.ginv);
+            // x^(1/g) = x/y^2 (y^(n-2) would carry n - 2 times y's error, and
+            // not the exponent that a rounded gamma asks for)
+            sol[0] = ROOT != 0 ? (y > 0. ? div64(rK * x, y * y) : 0.) : rK * pow(x, c.ginv);
         }
         sol[P] = p;
         vhalf = u - uK;

@@ -122,6 +122,7 @@ int sfx_solver_create(int kind, int ndim, double gamma, double tolerance, double
     c.rootf = (float)c.rn;
     const long double gl = gamma;
     c.rootk = c.root ? (float)(((gl - 1) / (2 * gl) - 1.0L / c.root) * std::log(2.0L)) : 0.f;
+    c.fank = c.root ? (float)((2 / (gl - 1) - (c.root - 2)) * std::log(2.0L)) : 0.f;
     c.kshock = std::sqrt(c.tdgp1 / gamma);
     hipError_t e = hipGetDevice(&h->device);
     if(e != hipSuccess) {

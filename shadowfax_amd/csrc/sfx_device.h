@@ -24,7 +24,8 @@ struct Consts {
     // (gamma = 7/5), else 0; 1/root and (1 + 1/root)/(2 root), its root
     // series; sqrt(2/(gamma (gamma+1)))
     int root;
-    float rootf, rootk;  // 1/root; ((g-1)/(2g) - 1/root) ln 2
+    // 1/root; ((g-1)/(2g) - 1/root) ln 2; (2/(g-1) - (root - 2)) ln 2
+    float rootf, rootk, fank;
     double rn, rn2, kshock;
 };
 
