@@ -156,7 +156,7 @@ __global__ __launch_bounds__(256) void drain_gradients(flux::MeshView<T> m, T* _
 
 template <int ND, int KIND, int MIXED, typename T, typename R, int ROOT>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(flux::face_waves<ND, KIND, MIXED>(), 10))) void drain_faces(flux::MeshView<T> m, const T* __restrict__ grad,
+__attribute__((amdgpu_waves_per_eu(flux::face_waves<ND, KIND, MIXED, ROOT>(), 10))) void drain_faces(flux::MeshView<T> m, const T* __restrict__ grad,
                                                    Consts cd, mixed::CF cf,
                                                    T* __restrict__ dQL,
                                                    uint8_t* __restrict__ fstatus,
@@ -211,7 +211,7 @@ __global__ __launch_bounds__(256) void range_gradients(flux::MeshView<T> m, T* _
 
 template <int ND, int KIND, int MIXED, typename T, typename R, int ROOT>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(flux::face_waves<ND, KIND, MIXED>(), 10))) void range_faces(flux::MeshView<T> m, const T* __restrict__ grad,
+__attribute__((amdgpu_waves_per_eu(flux::face_waves<ND, KIND, MIXED, ROOT>(), 10))) void range_faces(flux::MeshView<T> m, const T* __restrict__ grad,
                                                    Consts cd, mixed::CF cf,
                                                    T* __restrict__ dQL,
                                                    uint8_t* __restrict__ fstatus,

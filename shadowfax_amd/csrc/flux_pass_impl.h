@@ -1811,15 +1811,20 @@ __device__ __forceinline__ void face_item(const MeshView<T>& m, int64_t f,
 // general paths would otherwise set the register count (244 and 161; the
 // kernels' own code needs 150 and 110 in 3D); the others as they come.
 // (Mixed exact faces, 250,000 3D cells: 89 us at 4, 102 at 3, 162 at 5,
-// spilling; 2D, 262,144 cells: 29.7 at 6, 30.4 at 5, 31.2 at 4.)
-template <int ND, int KIND, int MIXED>
+// spilling; 2D, 262,144 cells: 29.7 at 6, 30.4 at 5, 31.2 at 4.  FP64 exact
+// faces of other gases, whose pow() spills at 4: gamma 1.66667, 150,001 2D cells
+// 55.4 us at 3, 65.5 at 4.)
+template <int ND, int KIND, int MIXED, int ROOT>
 constexpr int face_waves() {
-    return KIND != 0 ? 1 : MIXED == 0 ? (ND == 2 ? 4 : 3) : (ND == 2 ? 6 : 4);
+    if(KIND != 0) return 1;
+    if(MIXED == 0) return ND == 2 && ROOT != 0 ? 4 : 3;
+    return ND == 2 ? 6 : 4;
 }
 
 template <int ND, int KIND, int MIXED, typename T, typename R, bool FREC = false, int ROOT = 0>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(face_waves<ND, KIND, MIXED>(), 10))) void face_flux_kernel(MeshView<T> m, const T* __restrict__ grad,
+__attribute__((amdgpu_waves_per_eu(face_waves<ND, KIND, MIXED, ROOT>(), 10))) void face_flux_kernel(
+                                                        MeshView<T> m, const T* __restrict__ grad,
                                                         Consts cd, mixed::CF cf,
                                                         T* __restrict__ dQL,
                                                         uint8_t* __restrict__ fstatus,

@@ -17,11 +17,19 @@
 namespace sfx {
 namespace fp64 {
 
+// Waves per SIMD the kernels are held to: 4, and 3 for the exact solver of other
+// gases than 5/3 and 7/5, whose pow() spills at 4 (gamma 1.66667, 262,144 3D
+// problems: 115 us at 3, 123 at 4, 122 at 2; 2D 112, 123, 126).
+template <int KIND, int ROOT>
+constexpr int solver_waves() {
+    return KIND == 0 && ROOT == 0 ? 3 : 4;
+}
+
 // --------------------------------------------------------------- kernels --
 
 template <int ND, int KIND, int ROOT = 0>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void
-solve_for_flux_kernel(
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(solver_waves<KIND, ROOT>()))) void solve_for_flux_kernel(
         Consts c, int64_t N, const double* __restrict__ WL, const double* __restrict__ WR,
         const double* __restrict__ n, const double* __restrict__ v,
         const uint8_t* __restrict__ refl, double* __restrict__ F,
@@ -58,7 +66,8 @@ solve_for_flux_kernel(
 }
 
 template <int ND, int ROOT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void exact_solve_kernel(
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(solver_waves<0, ROOT>()))) void exact_solve_kernel(
         Consts c, int64_t N, const double* __restrict__ WL, const double* __restrict__ WR,
         const double* __restrict__ n, const uint8_t* __restrict__ refl,
         double* __restrict__ Whalf, double* __restrict__ WRout, double* __restrict__ mach_io,
@@ -97,7 +106,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void e
 // least bound caller, and they reserve as many (244 instead of 128: 262,144
 // problems 60 us instead of 47).
 template <int ND, int KIND, int ROOT, bool SOLVE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void scalar_kernel(
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(solver_waves<KIND, ROOT>()))) void scalar_kernel(
         Consts c, ScalarIn in, ScalarOut* __restrict__ out, unsigned long long* __restrict__ ctr) {
     if(threadIdx.x) return;
     unsigned iters = 0, brent = 0, vac = 0;
