@@ -108,7 +108,8 @@ int sfx_solver_enable_stats(sfx_solver* h, int enabled);
 int sfx_solver_set_split(sfx_solver* h, int iterations);
 int sfx_solver_get_split(const sfx_solver* h);
 
-/* ---- scalar drop-ins (host pointers, one problem on the GPU) --------- */
+/* ---- scalar drop-ins (host pointers, one problem on the GPU) ---------
+ * Several threads may call them on one handle: they take turns. */
 
 /* RiemannSolver::solve(WL, WR, n, mach, reflective)
  * (src/riemann/RiemannSolver.hpp:62-63, ExactRiemannSolver.cpp:108-290).

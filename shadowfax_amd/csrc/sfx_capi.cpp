@@ -380,6 +380,8 @@ static int scalar_run(sfx_solver* h, const double* WL, double* WR, const double*
     int rc = bind_device(h);
     if(rc) return rc;
     hipError_t e;
+    // (callers of one handle in several threads take turns)
+    std::lock_guard<std::mutex> lk(h->out_mu);
     if(!h->h_out) {
         e = hipHostMalloc((void**)&h->h_out, sizeof(ScalarOut),
                           hipHostMallocMapped | hipHostMallocCoherent);

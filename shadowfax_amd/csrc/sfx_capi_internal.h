@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdarg>
+#include <mutex>
 
 #include "sfx_device.h"
 
@@ -22,6 +23,7 @@ struct sfx_solver {
     sfx::ScalarOut* h_out = nullptr;      // scalar entry points: the result,
     sfx::ScalarOut* d_out = nullptr;      // pinned, and as the device sees it
     unsigned seq = 0;                     // the last scalar call's number
+    std::mutex out_mu;                    // held by the scalar call that uses these
     // work buffer (the straggler queue of the two-phase exact solve), grown
     // on demand
     void* d_scratch = nullptr;

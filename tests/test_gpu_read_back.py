@@ -54,3 +54,31 @@ def test_scalar_calls_equal_the_batch(device, nd, kind, precision):
     # the scalar calls are counted as the batch is
     n1 = s.stats()
     assert all(n1[k] == 2 * n0[k] for k in n0), (n0, n1)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_scalar_calls_of_several_threads(device, precision):
+    """Threads that solve on one handle each get their own problem's flux."""
+    import threading
+    import torch
+    T, N = 4, 200
+    b = WK.riemann_batch(T * N, seed=7, family="uniform", ndim=3)
+    t = lambda a: torch.tensor(np.ascontiguousarray(a), device=device)
+    s = RiemannSolver(0, 3, G, 1e-8, -5.0, precision)
+    F = s.solve_for_flux_batch(t(b["WL"]), t(b["WR"]), t(b["n"])).cpu().numpy()
+    got, errors = np.zeros_like(F), []
+
+    def work(k):
+        try:
+            for i in range(k * N, (k + 1) * N):
+                got[:, i] = s.solve_for_flux(b["WL"][:, i], b["WR"][:, i], b["n"][:, i])
+        except Exception as e:
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(T)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    assert not errors, errors
+    assert np.array_equal(got, F)
