@@ -375,7 +375,7 @@ __device__ __forceinline__ double limit1(double phimid0, double phiL, double phi
     double lim = far;
     if(!(far * phiL > 0.0)) {
         const double a = fabs(phiL);
-        lim = phiL * fp64::div64(a, fmax(a + delta1, 1e-300));
+        lim = phiL * fp64::div_any(a, a + delta1);
     }
     if(phiL == phiR) return phiL;
     if(up) return rmax(lim, rmin(phibar + delta2, phimid0));
@@ -1627,6 +1627,8 @@ __device__ __forceinline__ void face_item(const MeshView<T>& m, int64_t f,
         if(!skip) {
             solved = 1;
             R vface[ND];
+            R rRL2 = rr[0] * rr[0] + rr[1] * rr[1];
+            if(ND == 3) rRL2 = rr[0] * rr[0] + rr[1] * rr[1] + rr[ND - 1] * rr[ND - 1];
             if(!has_r) {
 #pragma unroll
                 for(int l = 0; l < ND; l++) vr[l] = R(0);
@@ -1638,15 +1640,13 @@ __device__ __forceinline__ void face_item(const MeshView<T>& m, int64_t f,
                     for(int l = 0; l < ND; l++) vr[l] = vl[l];
                     mirror_velocity<ND, R>(vr, rr);
                 }
-                R rRL2 = rr[0] * rr[0] + rr[1] * rr[1];
-                if(ND == 3) rRL2 = rr[0] * rr[0] + rr[1] * rr[1] + rr[ND - 1] * rr[ND - 1];
                 R fac = (vl[0] - vr[0]) * mcv[0];
                 fac += (vl[1] - vr[1]) * mcv[1];
                 if(ND == 3) fac += (vl[ND - 1] - vr[ND - 1]) * mcv[ND - 1];
                 if constexpr(MIXED)
                     fac *= mixed::rcp_nr(rRL2);
                 else
-                    fac = fp64::div64(fac, rRL2);
+                    fac = fp64::div_any(fac, rRL2);
 #pragma unroll
                 for(int l = 0; l < ND; l++) vface[l] = R(0.5) * (vl[l] + vr[l]) + fac * rr[l];
             } else {
@@ -1691,16 +1691,18 @@ __device__ __forceinline__ void face_item(const MeshView<T>& m, int64_t f,
                 for(int k = 0; k < NC; k++) WR[k] = WRrec[k];
             }
             // VorFace::get_normal (src/VorFace.cpp:553-571): n = -(xL - xR)/|xL - xR|
-            R nrm = (ND == 3) ? sqrt(rr[0] * rr[0] + rr[1] * rr[1] + rr[ND - 1] * rr[ND - 1])
-                              : sqrt(rr[0] * rr[0] + rr[1] * rr[1]);
             double flux[NC];
             if(!MIXED) {
                 double n64[ND], v64[ND], wl[NC], wr[NC];
-                const double inrm = fp64::rcp64((double)nrm);
+                const double nrm = sqrt((double)rRL2), inrm = fp64::rcp64(nrm);
 #pragma unroll
                 for(int l = 0; l < ND; l++) {
-                    n64[l] = fp64::div_by((double)rr[l], (double)nrm, inrm);
+                    n64[l] = fp64::div_by((double)rr[l], nrm, inrm);
                     v64[l] = (double)vface[l];
+                }
+                if(__builtin_expect(n64[0] != n64[0], 0)) {  // as div_any
+#pragma unroll
+                    for(int l = 0; l < ND; l++) n64[l] = (double)rr[l] / nrm;
                 }
 #pragma unroll
                 for(int k = 0; k < NC; k++) {
@@ -1747,20 +1749,11 @@ __device__ __forceinline__ void face_item(const MeshView<T>& m, int64_t f,
                 areaL = m.total_area[L];
                 areaR = m.total_area[Rs];
             }
-            // from reciprocals: a zero divisor gives NaN where a / b gives
-            // infinity, and no limit either way
             auto quot = [](double a, double b) {
                 if constexpr(MIXED)
                     return a * mixed::rcp_nr(b);
                 else
-                    return fp64::div64(a, b);
-            };
-            // a flux may be of any size
-            auto quot_any = [](double a, double b) {
-                if constexpr(MIXED)
-                    return a * mixed::rcp_nr(b);
-                else
-                    return a / b;
+                    return fp64::div_any(a, b);
             };
             double timefac = 1.;
             if(has_r) {
@@ -1771,7 +1764,7 @@ __device__ __forceinline__ void face_item(const MeshView<T>& m, int64_t f,
             double areafac = quot((double)A, areaL);
             areafac *= timefac;
             if(dQ[0] > areafac * massL) {
-                double corfac = fabs(quot_any(areafac * massL, dQ[0]));
+                double corfac = fabs(quot(areafac * massL, dQ[0]));
 #pragma unroll
                 for(int k = 0; k < NC; k++) dQ[k] *= corfac;
             }
@@ -1780,7 +1773,7 @@ __device__ __forceinline__ void face_item(const MeshView<T>& m, int64_t f,
                 af *= timefac;
                 // dQR[0] = -dQL[0]
                 if(-dQ[0] > af * massR) {
-                    double corfac = fabs(quot_any(af * massR, -dQ[0]));
+                    double corfac = fabs(quot(af * massR, -dQ[0]));
 #pragma unroll
                     for(int k = 0; k < NC; k++) dQ[k] = -(-dQ[k] * corfac);
                 }

@@ -24,8 +24,12 @@ namespace fp64 {
 // v_rcp_f64 and v_rsq_f64 give about 2^-24; one step of third order takes
 // that to the rounding error of the last two operations (about 1 ulp; half
 // an ulp with the residual's correction, div_by and sqrt64), in 4 to 9
-// instructions where the IEEE divide and square root take 12 and 22.  For x > 0 away from the ends of the exponent
-// range (no scaling): only ex_solve uses them, on the states it has tested.
+// instructions where the IEEE divide and square root take 12 and 22.  No
+// scaling: for operands away from the ends of the exponent range.  ex_solve,
+// root_setup (mixed) and the vacuum sides use them on states that they have
+// tested; hllc_solve_for_flux forms the sound speeds before its test, which is
+// false for the NaNs that come of others; the face predictor tests its density;
+// the face kernels' quotients by geometry, areas and times go through div_any.
 
 __device__ __forceinline__ double rcp64(double x) {
     const double r = __builtin_amdgcn_rcp(x);
@@ -38,6 +42,13 @@ __device__ __forceinline__ double div_by(double a, double b, double r) {
     return fma(fma(-b, q, a), r, q);
 }
 __device__ __forceinline__ double div64(double a, double b) { return div_by(a, b, rcp64(b)); }
+// a/b for any operands: where one is zero, infinite or at an end of the
+// exponent range, the steps above end as NaN and the IEEE quotient is taken
+__device__ __forceinline__ double div_any(double a, double b) {
+    double q = div64(a, b);
+    if(__builtin_expect(q != q, 0)) q = a / b;
+    return q;
+}
 // the correction of the estimate y of 1/sqrt(x), t = x y, in units of y
 __device__ __forceinline__ double rsq_step(double t, double y) {
     const double e = fma(-t, y, 1.0);

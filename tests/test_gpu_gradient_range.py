@@ -55,3 +55,39 @@ def test_gradients_bit_exact(device, nd, size, states):
     got = fp.m.grad_soa()
     assert np.array_equal(np.isnan(got), np.isnan(ref))
     assert np.array_equal(got, ref, equal_nan=True)
+
+
+@pytest.mark.parametrize("nd,size", [(2, 0), (3, 0), (2, -400), (3, 400), (2, -520), (2, 520),
+                                     (3, -508)])
+@pytest.mark.parametrize("kind", [0, 1])
+def test_faces_of_any_size(device, nd, size, kind):
+    """FP64 face fluxes of meshes whose squared lengths are in, below (down to
+    subnormal) and above the range of the shared reciprocals: the oracle's to
+    1e-11 normwise (its fluxes' 1e-12, ten quotients in a row), and infinity
+    and NaN where it has them."""
+    import torch
+    print("case", nd, size, kind, flush=True)
+    rng = np.random.default_rng(9)
+    W = rng.uniform(0.5, 2.0, (nd + 2, 300))
+    W[1:-1] -= 1.0
+    with np.errstate(all="ignore"):
+        m = scaled(M.voronoi_periodic(M.poisson_points(300, seed=5, ndim=nd)),
+                   np.float64(2.0) ** size)
+        b = M.prepare(m, W, G, kind=kind, vel=rng.uniform(-1, 1, (nd, 300)), dt=1e-3)
+        b["mass"] = np.ones(300)  # the large meshes' fluxes meet the mass limiter
+        ob = dict(b, grad=np.zeros((nd, nd + 2, 300)))
+        _, ref, _, _ = O.face_flux_pass(kind, ob)
+    s = RiemannSolver(kind, nd, G, 1e-8, -5.0, "fp64")
+    fp = FluxPass(s, M.DeviceMesh(b, "fp64", device))
+    fp.m.grad.zero_()
+    fp.face_fluxes()
+    torch.cuda.synchronize()
+    got = fp.m.dQL_soa()
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    ok = np.isfinite(ref).all(0)
+    assert np.array_equal(got[:, ~ok], ref[:, ~ok], equal_nan=True)
+    err = np.abs(got - ref)[:, ok].max(0)
+    scale = np.abs(ref)[:, ok].max(0)
+    print("faces %d of %d, max %.2e" % (ok.sum(), len(ok), (err / scale)[scale > 1e-300].max()
+                                        if (scale > 1e-300).any() else 0.0), flush=True)
+    assert ok.any() and (err <= 1e-11 * scale + 1e-320).all()
