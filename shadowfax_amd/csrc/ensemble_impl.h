@@ -154,9 +154,23 @@ __global__ __launch_bounds__(256) void drain_gradients(flux::MeshView<T> m, T* _
     });
 }
 
+// Waves per SIMD the face drains are held to: as the standalone kernels but for
+// mixed exact faces in 2D, which spill 91 registers at 6, and FP64 exact ones in
+// 3D (171 at 3).  (Steps of 16 meshes of 4,900 2D or 2,744 3D cells: mixed exact
+// 2D 66.4 us at 4, 70.9 at 5, 73.2 at 6, 78.6 at 3; FP64 exact 3D 128 at 2, 139
+// at 3, 2D 85.6 at 4, 89.2 at 3; FP64 HLLC 2D 78.6 at 4, 86.1 unbound, 3D 117 at
+// 3, 127 unbound, 142 at 4.)
+template <int ND, int KIND, int MIXED, int ROOT>
+constexpr int drain_waves() {
+    if(KIND == 0 && MIXED != 0) return 4;
+    if(KIND == 0 && ND == 3) return 2;
+    return flux::face_waves<ND, KIND, MIXED, ROOT>();
+}
+
 template <int ND, int KIND, int MIXED, typename T, typename R, int ROOT>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(flux::face_waves<ND, KIND, MIXED, ROOT>(), 10))) void drain_faces(flux::MeshView<T> m, const T* __restrict__ grad,
+__attribute__((amdgpu_waves_per_eu(drain_waves<ND, KIND, MIXED, ROOT>(), 10))) void drain_faces(
+                                                   flux::MeshView<T> m, const T* __restrict__ grad,
                                                    Consts cd, mixed::CF cf,
                                                    T* __restrict__ dQL,
                                                    uint8_t* __restrict__ fstatus,
@@ -211,7 +225,8 @@ __global__ __launch_bounds__(256) void range_gradients(flux::MeshView<T> m, T* _
 
 template <int ND, int KIND, int MIXED, typename T, typename R, int ROOT>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(flux::face_waves<ND, KIND, MIXED, ROOT>(), 10))) void range_faces(flux::MeshView<T> m, const T* __restrict__ grad,
+__attribute__((amdgpu_waves_per_eu(flux::face_waves<ND, KIND, MIXED, ROOT>(), 10))) void range_faces(
+                                                   flux::MeshView<T> m, const T* __restrict__ grad,
                                                    Consts cd, mixed::CF cf,
                                                    T* __restrict__ dQL,
                                                    uint8_t* __restrict__ fstatus,

@@ -1802,14 +1802,16 @@ __device__ __forceinline__ void face_item(const MeshView<T>& m, int64_t f,
 
 // Waves per SIMD a face kernel is held to: the exact solvers' out-of-line
 // general paths would otherwise set the register count (244 and 161; the
-// kernels' own code needs 150 and 110 in 3D); the others as they come.
+// kernels' own code needs 150 and 110 in 3D); FP64 HLLC to what its standalone
+// kernels have, which the ensembles' drains around it would exceed; mixed HLLC as
+// it comes.
 // (Mixed exact faces, 250,000 3D cells: 89 us at 4, 102 at 3, 162 at 5,
 // spilling; 2D, 262,144 cells: 29.7 at 6, 30.4 at 5, 31.2 at 4.  FP64 exact
 // faces of other gases, whose pow() spills at 4: gamma 1.66667, 150,001 2D cells
 // 55.4 us at 3, 65.5 at 4.)
 template <int ND, int KIND, int MIXED, int ROOT>
 constexpr int face_waves() {
-    if(KIND != 0) return 1;
+    if(KIND != 0) return MIXED != 0 ? 1 : ND == 2 ? 4 : 3;
     if(MIXED == 0) return ND == 2 && ROOT != 0 ? 4 : 3;
     return ND == 2 ? 6 : 4;
 }
