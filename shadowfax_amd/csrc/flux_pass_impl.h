@@ -173,7 +173,7 @@ struct Rec64 {
 // is an estimate of 1/b, two Newton steps, the product and its residual's
 // correction, wrapped in a scaling of operands near the ends of the exponent
 // range and a fix-up of zeros, infinities and NaNs (12 instructions).  For
-// operands that are zero or within 2^-200 .. 2^200 neither wrapper changes
+// operands that are zero or in quot_wide's ranges neither wrapper changes
 // anything, and quotients by the same b share its reciprocal: 3 instructions
 // each (a zero quotient may lose a minus sign).
 struct Recip {
@@ -188,10 +188,16 @@ __device__ __forceinline__ double quot_by(double a, const Recip& d) {
     const double q = a * d.r;
     return fma(fma(-d.b, q, a), d.r, q);
 }
-// x is neither zero (or below 2^-1042) nor within 2^-200 .. 2^200
+// x is neither zero (or below 2^-1042) nor within 2^-E .. 2^E.  E = 200 for the
+// geometry; the states, which enter the quotients once, may lie within 2^-500 ..
+// 2^500 then: a difference of two is at least 2^-552, its quotient 2^-952, with
+// its residual far from underflow.  (The tail of a Gaussian perturbation reaches
+// 1e-100 easily: at 200 for the states too, velocities of 1e-80 took the 3D
+// gradients of 120,000 cells from 66 to 135 us.)
+template <int E>
 __device__ __forceinline__ bool quot_wide(double x) {
     const uint32_t u = (uint32_t)(__double_as_longlong(x) >> 32) & 0x7fffffffu;
-    return u > ((1023u + 200u) << 20) || u - 1u < ((1023u - 200u) << 20);
+    return u > ((1023u + E) << 20) || u - 1u < ((1023u - E) << 20);
 }
 
 // Row o of an item-major FP64 array of NC = 4 or 5 values per item
@@ -701,7 +707,7 @@ __device__ __forceinline__ void entry_record_from_vals64(const EntryVals64<ND>& 
         rec[RL::D + l] = v.area != 0.0 ? v.d[l] : 0.0;
         rec[RL::C + l] = v.mc[l];
         rec[RL::R + l] = isR ? v.rRL[l] : -v.rRL[l];
-        wide |= quot_wide(v.mc[l]) | quot_wide(v.rRL[l]);
+        wide |= quot_wide<200>(v.mc[l]) | quot_wide<200>(v.rRL[l]);
     }
     bool zero = true;
 #pragma unroll
@@ -1258,7 +1264,7 @@ __device__ __forceinline__ void grad_cell_f64(const MeshView<T>& m, int64_t s,
     const R V = (R)m.volume[i];
     bool ieee = false;  // an operand out of quot_by's range
 #pragma unroll
-    for(int k = 0; k < NC; k++) ieee |= quot_wide(W[k]);
+    for(int k = 0; k < NC; k++) ieee |= quot_wide<500>(W[k]);
     if(!act) n = 0;
     // the cell's records as positions n - 1 .. 0 (reverse walk order,
     // src/VorCell.cpp:471): entries base + p, or rows base + p of the
@@ -1271,97 +1277,97 @@ __device__ __forceinline__ void grad_cell_f64(const MeshView<T>& m, int64_t s,
     // unconditionally: a mirror neighbour is the cell's own row, reflected
     // afterwards), so a lane has KB independent loads in flight
     constexpr int KB = SFX_GRAD_KB;
-    for(int64_t pb = n; pb > 0; pb -= KB) {
-        R A[KB], c[KB][ND], rij[KB][ND], Wj[KB][NC];
-        int32_t o[KB];
-        bool wide[KB];
+    // divide: IEEE quotients for every face
+    const auto sums = [&](auto divide) {
+        for(int64_t pb = n; pb > 0; pb -= KB) {
+            R A[KB], c[KB][ND], rij[KB][ND], Wj[KB][NC];
+            int32_t o[KB];
+            bool wide[KB];
 #pragma unroll
-        for(int u = 0; u < KB; u++) {
-            const int64_t p = pb - 1 - u;
-            alignas(16) T rec[ER];
-            load_record<ND, T, GROUPED>(m, base, p >= 0 ? p : 0, lane, rec);
-            A[u] = rec[RL::A];
+            for(int u = 0; u < KB; u++) {
+                const int64_t p = pb - 1 - u;
+                alignas(16) T rec[ER];
+                load_record<ND, T, GROUPED>(m, base, p >= 0 ? p : 0, lane, rec);
+                A[u] = rec[RL::A];
 #pragma unroll
-            for(int l = 0; l < ND; l++) {
-                c[u][l] = rec[RL::C + l];
-                rij[u][l] = rec[RL::R + l];
+                for(int l = 0; l < ND; l++) {
+                    c[u][l] = rec[RL::C + l];
+                    rij[u][l] = rec[RL::R + l];
+                }
+                o[u] = bits_index(rec[RL::NB]);
+                wide[u] = (__double_as_longlong(rec[RL::NB]) >> 32) != 0;
             }
-            o[u] = bits_index(rec[RL::NB]);
-            wide[u] = (__double_as_longlong(rec[RL::NB]) >> 32) != 0;
-        }
 #pragma unroll
-        for(int u = 0; u < KB; u++) {
-            const int64_t src = o[u] >= 0 ? (int64_t)o[u] : i;
+            for(int u = 0; u < KB; u++) {
+                const int64_t src = o[u] >= 0 ? (int64_t)o[u] : i;
 #pragma unroll
-            for(int k = 0; k < NC; k++) Wj[u][k] = (R)m.W[src * NC + k];
-        }
+                for(int k = 0; k < NC; k++) Wj[u][k] = (R)m.W[src * NC + k];
+            }
 #pragma unroll
-        for(int u = 0; u < KB; u++) {
-            if(o[u] < 0) {
-                // mirror neighbour (:482-489); only a left cell has one, so
-                // rRL = -r_ij
-                R rr[ND];
+            for(int u = 0; u < KB; u++) {
+                if(o[u] < 0) {
+                    // mirror neighbour (:482-489); only a left cell has one, so
+                    // rRL = -r_ij
+                    R rr[ND];
 #pragma unroll
-                for(int l = 0; l < ND; l++) rr[l] = -rij[u][l];
-                mirror_velocity<ND, R>(Wj[u] + 1, rr);
+                    for(int l = 0; l < ND; l++) rr[l] = -rij[u][l];
+                    mirror_velocity<ND, R>(Wj[u] + 1, rr);
+                }
+            }
+#pragma unroll
+            for(int u = 0; u < KB; u++) {
+                if(u >= pb || !(A[u] != R(0))) continue;  // also the padding
+                const R rnorm =
+                        (ND == 3) ? sqrt(rij[u][0] * rij[u][0] + rij[u][1] * rij[u][1] +
+                                         rij[u][ND - 1] * rij[u][ND - 1])
+                                  : sqrt(rij[u][0] * rij[u][0] + rij[u][1] * rij[u][1]);
+#pragma unroll
+                for(int k = 0; k < NC; k++) wide[u] |= quot_wide<500>(Wj[u][k]);
+                // in 2D IEEE quotients per face; in 3D, where the branch would cost
+                // a wave per SIMD (203 registers, 8 of 145 us), the cell's sums
+                // again below.  (Velocities with a Gaussian tail to 1e-305, 22% of
+                // the cells beyond 2^-500: 2D, 150,001 cells, 33 us, with the sums
+                // again 38; 3D, 120,000 cells, 112 us, a face at a time 125.)
+                const auto by_divide = [&] {
+#pragma unroll
+                    for(int l = ND; l--;)
+#pragma unroll
+                        for(int k = 0; k < NC; k++)
+                            delta[l][k] += A[u] * ((Wj[u][k] - W[k]) * c[u][l] / rnorm -
+                                                   R(0.5) * (W[k] + Wj[u][k]) * rij[u][l] / rnorm);
+                };
+                if constexpr(decltype(divide)::value) {
+                    by_divide();
+                    continue;
+                }
+                ieee |= ND == 3 && wide[u];
+                if(ND == 2 && __builtin_expect(ieee | wide[u], 0)) {
+                    by_divide();
+                } else {
+                    const Recip rn = recip_of(rnorm);
+#pragma unroll
+                    for(int l = ND; l--;)
+#pragma unroll
+                        for(int k = 0; k < NC; k++)
+                            delta[l][k] +=
+                                    A[u] * (quot_by((Wj[u][k] - W[k]) * c[u][l], rn) -
+                                            quot_by(R(0.5) * (W[k] + Wj[u][k]) * rij[u][l], rn));
+                }
+#pragma unroll
+                for(int k = 0; k < NC; k++) {
+                    Wmax[k] = smaxr<R>(Wmax[k], Wj[u][k]);
+                    Wmin[k] = sminr<R>(Wmin[k], Wj[u][k]);
+                }
             }
         }
-#pragma unroll
-        for(int u = 0; u < KB; u++) {
-            if(u >= pb || !(A[u] != R(0))) continue;  // also the padding
-            const R rnorm =
-                    (ND == 3) ? sqrt(rij[u][0] * rij[u][0] + rij[u][1] * rij[u][1] +
-                                     rij[u][ND - 1] * rij[u][ND - 1])
-                              : sqrt(rij[u][0] * rij[u][0] + rij[u][1] * rij[u][1]);
-#pragma unroll
-            for(int k = 0; k < NC; k++) wide[u] |= quot_wide(Wj[u][k]);
-            ieee |= wide[u];
-            const Recip rn = recip_of(rnorm);
-#pragma unroll
-            for(int l = ND; l--;)
-#pragma unroll
-                for(int k = 0; k < NC; k++)
-                    delta[l][k] += A[u] * (quot_by((Wj[u][k] - W[k]) * c[u][l], rn) -
-                                           quot_by(R(0.5) * (W[k] + Wj[u][k]) * rij[u][l], rn));
-#pragma unroll
-            for(int k = 0; k < NC; k++) {
-                Wmax[k] = smaxr<R>(Wmax[k], Wj[u][k]);
-                Wmin[k] = sminr<R>(Wmin[k], Wj[u][k]);
-            }
-        }
-    }
-    if(ieee) {
-        // the sums again, a face at a time, with IEEE quotients
+    };
+    sums(std::false_type());
+    if(ND == 3 && ieee) {
 #pragma unroll
         for(int l = 0; l < ND; l++)
 #pragma unroll
             for(int k = 0; k < NC; k++) delta[l][k] = R(0);
-        for(int64_t p = n - 1; p >= 0; p--) {
-            alignas(16) T rec[ER];
-            load_record<ND, T, GROUPED>(m, base, p, lane, rec);
-            if(!(rec[RL::A] != R(0))) continue;
-            const int32_t o = bits_index(rec[RL::NB]);
-            R Wj[NC], r2 = R(0);
-#pragma unroll
-            for(int k = 0; k < NC; k++) Wj[k] = m.W[(o >= 0 ? (int64_t)o : i) * NC + k];
-            if(o < 0) {
-                R rr[ND];
-#pragma unroll
-                for(int l = 0; l < ND; l++) rr[l] = -rec[RL::R + l];
-                mirror_velocity<ND, R>(Wj + 1, rr);
-            }
-#pragma unroll
-            for(int l = 0; l < ND; l++) r2 = l ? r2 + rec[RL::R + l] * rec[RL::R + l]
-                                               : rec[RL::R] * rec[RL::R];
-            const R rnorm = sqrt(r2);
-#pragma unroll
-            for(int l = ND; l--;)
-#pragma unroll
-                for(int k = 0; k < NC; k++)
-                    delta[l][k] += rec[RL::A] *
-                                   ((Wj[k] - W[k]) * rec[RL::C + l] / rnorm -
-                                    R(0.5) * (W[k] + Wj[k]) * rec[RL::R + l] / rnorm);
-        }
+        sums(std::true_type());
     }
 #pragma unroll
     for(int l = ND; l--;)

@@ -91,3 +91,31 @@ def test_faces_of_any_size(device, nd, size, kind):
     print("faces %d of %d, max %.2e" % (ok.sum(), len(ok), (err / scale)[scale > 1e-300].max()
                                         if (scale > 1e-300).any() else 0.0), flush=True)
     assert ok.any() and (err <= 1e-11 * scale + 1e-320).all()
+
+
+@pytest.mark.parametrize("nd", [2, 3])
+@pytest.mark.parametrize("size", [0, -190, 190])
+def test_gradients_of_extreme_states(device, nd, size):
+    """States near the ends of their range (2^-500 .. 2^500) and beyond, each
+    component another power of two and a tail that falls through the whole
+    range to subnormals and zero, bit for bit the oracle's."""
+    import torch
+    m = scaled(M.voronoi_periodic(M.poisson_points(300, seed=5, ndim=nd)), 2.0 ** size)
+    rng = np.random.default_rng(11)
+    for powers in ((-495, -505, 0, -90), (495, 480, 0, 300), (-600, 0, 490, -499)):
+        print("case", nd, size, powers, flush=True)
+        W = rng.uniform(0.5, 2.0, (nd + 2, 300))
+        for k, e in enumerate(powers):
+            W[k] *= 2.0 ** e
+        W[1] *= rng.choice([-1.0, 1.0], 300)
+        W[2, ::2] *= np.exp(-rng.uniform(0, 28, 150) ** 2)
+        with np.errstate(all="ignore"):
+            b = M.prepare(m, W, G, kind=0, vel=np.zeros((nd, 300)), dt=1e-3)
+            ref = O.gradients(0, b)
+        fp = FluxPass(RiemannSolver(0, nd, G, 1e-8, -5.0, "fp64"),
+                      M.DeviceMesh(b, "fp64", device))
+        fp.gradients()
+        torch.cuda.synchronize()
+        got = fp.m.grad_soa()
+        assert np.array_equal(np.isnan(got), np.isnan(ref))
+        assert np.array_equal(got, ref, equal_nan=True)
