@@ -671,7 +671,7 @@ __device__ __forceinline__ void root_setup(const CF& c, const Consts& cd, bool r
     // any unit will do; false for NaNs too
     const double rmax = fmax(rL, rR), pmin = fmin(pL, pR), pmax = fmax(pL, pR);
     if(!(rL >= 1e-100 && rR >= 1e-100 && pL >= 1e-100 && pR >= 1e-100 && rmax <= 1e100 &&
-         pmax <= 1e100 && pmax <= 1e18 * pmin)) {
+         pmax <= 1e100 && pmax <= 1e30 * pmin)) {
         s.phase = EX_GENERAL;
         // vacuum beside such a gas, or on both sides: closed forms here (out of
         // line 1,048,576 problems took 169 us, 16 here)
@@ -698,10 +698,10 @@ __device__ __forceinline__ void root_setup(const CF& c, const Consts& cd, bool r
     s.pure_newton = dud - (taLd + taRd) < cd.cutoff;
     const float aL = (float)s.aLd, aR = (float)s.aRd;
     const float du = (float)dud, taL = (float)taLd, taR = (float)taRd;
-    // the ram pressure: p* is at most 2 (pmax + ram), 4e24 pmin
+    // the ram pressure: p* is at most 2 (pmax + ram), 4e30 pmin
     const double ram = rmax * dud * dud;
     const float amin = fminf(aL, aR), amax = fmaxf(aL, aR);
-    if(!(ram <= 1e24 * pmin && amax <= 1e8f * amin && amin >= 1e-25f && amax <= 1e20f)) {
+    if(!(ram <= 1e30 * pmin && amax <= 1e15f * amin && amin >= 1e-25f && amax <= 1e20f)) {
         s.phase = EX_GENERAL;
         return;
     }
@@ -724,8 +724,15 @@ __device__ __forceinline__ void root_setup(const CF& c, const Consts& cd, bool r
         const float k = (float)cd.kshock;
         const float gL = k * aL * __builtin_amdgcn_rsqf(xpv + c.gm1dgp1),
                     gR = k * aR * __builtin_amdgcn_rsqf(xpv * rx + c.gm1dgp1);
-        // (far from the truth where a light side meets a heavy one)
-        xg = fminf((gL + gR - du) * rcpf(gL + gR * rx), (float)(2.0 * (pmax + ram) * ipL));
+        // far from the truth where a light side meets a heavy one; but each
+        // side's share of the pressure function is at most the other's 2 a/(g-1)
+        // less du, and a shock's is that at less than 2 (p + rho (its share)^2).
+        // (Not for the pure Newton scheme, whose outcome depends on its guess:
+        // far right of the root it ends at p* = 0.)
+        const double eL = taRd - dud, eR = taLd - dud;
+        double cap = pmax + ram;
+        if(!s.pure_newton) cap = fmin(cap, fmin(fma(rL * eL, eL, pL), fma(rR * eR, eR, pR)));
+        xg = fminf((gL + gR - du) * rcpf(gL + gR * rx), (float)(2.0 * cap * ipL));
     }
     s.z = exp2f_fast(cd.rootf * log2f_fast(fmaxf(xfloor, xg)));
 }

@@ -158,3 +158,40 @@ def test_split_equals_one_kernel_over_the_range(device, gamma, nd):
     for F, st, c in out[1:]:
         assert np.array_equal(F, out[0][0], equal_nan=True)
         assert np.array_equal(st, out[0][1]) and c == out[0][2]
+
+
+@pytest.mark.parametrize("nd", [2, 3])
+@pytest.mark.parametrize("gamma", [5.0 / 3.0, 1.4])
+def test_mixed_exact_pressure_ratios(device, gamma, nd):
+    """Pressure ratios from 1e15 to the limit of the iteration in the n-th
+    root (1e30), each way, with streams that collide and separate."""
+    import torch
+    print("case", gamma, nd, flush=True)
+    N = 6000
+    b = WK.riemann_batch(N, seed=47, family="uniform", ndim=nd, round32=False)
+    WL, WR, n = b["WL"], b["WR"], b["n"]
+    r = np.random.RandomState(47)
+    ratio = 10.0 ** r.uniform(15, 29.9, N)
+    up = r.uniform(size=N) < 0.5
+    WL[-1] = np.where(up, 1e10, 1e10 / ratio)
+    WR[-1] = np.where(up, 1e10 / ratio, 1e10)
+    # the low side's density from the high one's towards where the sound speeds
+    # are alike
+    lo = 10.0 ** r.uniform(-14, 0, N)
+    lo[::3] = 10.0 ** r.uniform(-2, 2, len(lo[::3]))  # alike: a cold side beside a hot one
+    WL[0], WR[0] = np.where(up, WL[0], WR[0] * lo), np.where(up, WL[0] * lo, WR[0])
+    a = np.sqrt(1e10 / np.maximum(WL[0], WR[0]))
+    s = r.uniform(-3, 1, N) * a
+    WL[1:-1] += s * n
+    t = lambda a: torch.tensor(np.ascontiguousarray(a), device=device)
+    out = {}
+    for prec in ("fp64", "mixed"):
+        s = RiemannSolver(0, nd, gamma, 1e-8, -5.0, prec)
+        st = torch.zeros(N, dtype=torch.uint8, device=device)
+        F = s.solve_for_flux_batch(t(WL), t(WR), t(n), status=st)
+        torch.cuda.synchronize()
+        out[prec] = (F.cpu().numpy(), st.cpu().numpy())
+    assert np.array_equal(out["mixed"][1], out["fp64"][1])
+    err = normwise_error(out["mixed"][0], out["fp64"][0], WL, WR, gamma)
+    print("max %.2e" % err.max(), flush=True)
+    assert err.max() <= TOL
