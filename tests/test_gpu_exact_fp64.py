@@ -7,7 +7,8 @@ the step-by-step path runs, walls and moving faces.
 Tolerance: both iterations take the same steps and tests; Brent's method may
 stop up to 1e-8 from the root, and where it does so, round-off in the pressure
 function moves its last iterates by a multiple of that round-off (1e-16)
-that grows with the number of steps: 1e-10 normwise leaves six decades."""
+that grows with the number of steps: 1e-10 normwise leaves six decades.  Newton's
+method ends within round-off of the root: 1e-12, as for the fluxes in general."""
 import numpy as np
 import pytest
 
@@ -18,12 +19,14 @@ from shadowfax_amd.riemann import RiemannSolver
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-10
+TOL_NEWTON = 1e-12
 
 
 def edge_batch(nd, seed):
     """The mixed family, then blocks of it rescaled: pressures 1e10 to 1e13
-    apart each way (ratios to 1e26: the limit is 1e24), densities around
-    1e-100, colliding and separating streams, and equal states."""
+    apart each way (ratios to 1e26: the limit is 1e24), densities and pressures
+    around 1e-100 and 1e100, colliding and separating streams, and equal
+    states."""
     b = WK.riemann_batch(6000, seed=seed, family="mixed", ndim=nd, round32=False)
     WL, WR, n = b["WL"], b["WR"], b["n"]
     u = np.random.RandomState(seed).uniform(size=6000)
@@ -31,8 +34,11 @@ def edge_batch(nd, seed):
     m = (k >= 2000) & (k < 3000)
     WL[-1, m] *= 10.0 ** (10 + 3 * u[m])
     WR[-1, m] *= 10.0 ** -(10 + 3 * u[m])
-    m = (k >= 3000) & (k < 3500)
-    WL[0, m] = 1e-100 * (0.5 + u[m])
+    for lo, f in ((3000, 1e-100), (3250, 1e100)):  # sound speeds unchanged
+        m = (k >= lo) & (k < lo + 250)
+        for W in (WL, WR):
+            W[0, m] *= f
+            W[-1, m] *= f
     m = (k >= 3500) & (k < 4000)
     WR[:, m] = WL[:, m]
     m = (k >= 4000) & (k < 5000)
@@ -66,21 +72,23 @@ def test_exact_fp64_matches_step_by_step(device, gamma, nd):
         Fo, sto, c = O.solve_for_flux(O.EXACT, nd, WL, WR, n, v=v, refl=refl, gamma=gamma)
         Wo = O.exact_solve(nd, WL, WR, n, refl=refl, gamma=gamma)[0]
         err = normwise_error(F.cpu().numpy(), Fo, WL, WR, gamma)
-    # sides whose sound speeds are more than 1/eps apart (the 1e-100
-    # densities) run the step-by-step path, as all that are 1e8 apart; its
-    # answer there is the fast side's round-off, and the device's pow() and
-    # glibc's give fluxes that differ by factors
-    a = np.sqrt(np.maximum(WL[-1] / WL[0], WR[-1] / WR[0]) /
-                np.minimum(WL[-1] / WL[0], WR[-1] / WR[0]))
-    same = a <= 1e16
-    assert same[:2000].all() and not same[3000:3500].any() and same[3500:].all()
-    assert np.array_equal((st.cpu().numpy() != 0)[same], (sto != 0)[same])
-    ok = same & (sto == 0) & np.isfinite(Fo).all(0)
+    assert np.array_equal(st.cpu().numpy() != 0, sto != 0)
+    ok = (sto == 0) & np.isfinite(Fo).all(0)
     scale = np.maximum(np.abs(WL), np.abs(np.where(refl, WL, WR))).max(0)
     eh = (np.abs(Wh.cpu().numpy() - Wo) / np.maximum(scale, np.abs(Wo).max(0))).max(0)
-    print("flux %.2e half state %.2e" % (err[ok].max(), eh[ok].max()), flush=True)
-    assert ok.mean() > 0.9
+    # without Brent's method, and without streams that collide at up to 1e4 sound
+    # speeds, whose momenta cancel, both iterations end at the root
+    brent = np.array([O.solve_for_flux(O.EXACT, nd, WL[:, i:i + 1], WR[:, i:i + 1], n[:, i:i + 1],
+                                       v=v[:, i:i + 1], refl=refl[i:i + 1],
+                                       gamma=gamma)[2].nbrent for i in range(N)])
+    k = np.arange(N)
+    newton = ok & (brent == 0) & ((k < 2000) | ((k >= 3500) & (k < 4000)) | (k >= 5000))
+    print("flux %.2e half state %.2e, Newton's alone %.2e %.2e" % (
+        err[ok].max(), eh[ok].max(), err[newton].max(), eh[newton].max()), flush=True)
+    assert ok.mean() > 0.9 and newton.sum() > 2500
     assert err[ok].max() <= TOL and eh[ok].max() <= TOL
+    if gamma >= 1.4:  # (1.05: near vacuum the steps shrink too slowly to tell the root)
+        assert err[newton].max() <= TOL_NEWTON and eh[newton].max() <= TOL_NEWTON
     assert s.stats()["nvacuum"] == 2 * c.nvacuum
 
 
