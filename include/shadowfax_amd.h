@@ -371,10 +371,10 @@ typedef struct {
                                   (sfx_cell_closure); NULL when the cells'
                                   faces close, as those of a Voronoi
                                   tessellation do */
-    const void* frec;          /* float4 [sfx_mesh_face_record_planes(...)][F]
+    const void* frec;          /* sfx_mesh_face_record_planes(...) F float4
                                   or NULL (mixed pass only): the faces' own
-                                  values packed by sfx_mesh_face_records,
-                                  16-byte aligned; the face kernel then reads
+                                  values packed by sfx_mesh_face_records in
+                                  its order, 16-byte aligned; the face kernel then reads
                                   them instead of left, right, area, dL, dR,
                                   rRL, mc and rcent (which stay required) */
 } sfx_mesh;
@@ -416,8 +416,8 @@ int sfx_mesh_entry_record(int ndim, int precision);
  *   2D: [left, right, area, rcent] [rRL (2), mc (2)] [dL (2), dR (2)]
  * with left and right as their int32 bits.  The face kernel then loads a
  * face with 3 or 4 16-byte reads instead of 13 or 17 4-byte ones; the
- * fluxes are bit for bit the same.  frec: float4 [planes][F], 16-byte
- * aligned.  Mixed-precision handles only (SFX_ERR_ARG otherwise). */
+ * fluxes are bit for bit the same.  frec: P F float4 in that order,
+ * 16-byte aligned.  Mixed-precision handles only (SFX_ERR_ARG otherwise). */
 int sfx_mesh_face_records(sfx_solver* h, const sfx_mesh* m, void* frec, void* stream);
 
 /* float4 planes per face record: 4 (3D) or 3 (2D) for the mixed precision,

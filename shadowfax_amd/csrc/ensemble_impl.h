@@ -187,13 +187,11 @@ __attribute__((amdgpu_waves_per_eu(drain_waves<ND, KIND, MIXED, ROOT>(), 10))) v
 template <int ND, int MIXED, typename T>
 __global__ __launch_bounds__(256) void drain_gather(const int64_t* __restrict__ goff,
                                                     const int32_t* __restrict__ gent,
-                                                    const uint8_t* __restrict__ ghost,
-                                                    const int32_t* __restrict__ twin,
                                                     const T* __restrict__ dQL,
                                                     double* __restrict__ dQ,
                                                     Plan* __restrict__ p, int grid) {
     drain<false>(p, 2, grid, [&](const Slot& sl, int64_t i) {
-        flux::gather_cell<ND, MIXED, T>(i, goff, gent, ghost, twin, dQL, sl.qshift, dQ);
+        flux::gather_cell<ND, MIXED, T>(i, goff, gent, dQL, sl.qshift, dQ);
     });
 }
 
@@ -244,14 +242,12 @@ __attribute__((amdgpu_waves_per_eu(flux::face_waves<ND, KIND, MIXED, ROOT>(), 10
 template <int ND, int MIXED, typename T>
 __global__ __launch_bounds__(256) void range_gather(const int64_t* __restrict__ goff,
                                                     const int32_t* __restrict__ gent,
-                                                    const uint8_t* __restrict__ ghost,
-                                                    const int32_t* __restrict__ twin,
                                                     const T* __restrict__ dQL,
                                                     double* __restrict__ dQ, int64_t cell0,
                                                     int64_t ncell, int64_t qshift) {
     const int64_t k = xcd_block() * blockDim.x + threadIdx.x;
     if(k < ncell)
-        flux::gather_cell<ND, MIXED, T>(cell0 + k, goff, gent, ghost, twin, dQL, qshift, dQ);
+        flux::gather_cell<ND, MIXED, T>(cell0 + k, goff, gent, dQL, qshift, dQ);
 }
 
 template <int ND>

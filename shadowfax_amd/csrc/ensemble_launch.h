@@ -34,7 +34,7 @@ hipError_t ens_step_impl(int ndim, int kind, const EnsArgs<T>& a, hipStream_t s)
             hipLaunchKernelGGL((ens::drain_faces<ND, 1, MIXED, T, double, 0>), gf, b, 0, s,     \
                                a.m, a.grad, a.c, cf, a.dQL, a.fstatus, a.ctr, a.plan, grid);    \
         hipLaunchKernelGGL((ens::drain_gather<ND, MIXED, T>), gc, b, 0, s, a.m.gather_off,         \
-                           a.m.gather_entry, a.m.ghost, a.m.twin, a.dQL, a.dQ, a.plan, grid);   \
+                           a.m.gather_entry, a.dQL, a.dQ, a.plan, grid);                       \
         hipLaunchKernelGGL((ens::drain_update<ND>), gc, b, 0, s, a.c, a.Q, a.dQ, a.m.volume,    \
                            a.W, a.cstatus, a.mass, a.ctr, a.plan, grid);                        \
     } while(0)
@@ -72,7 +72,7 @@ hipError_t ens_range_impl(int ndim, int kind, const EnsArgs<T>& a, int64_t cell0
                                    nface, gshift, qshift);                                      \
         }                                                                                      \
         hipLaunchKernelGGL((ens::range_gather<ND, MIXED, T>), gc, b, 0, s, a.m.gather_off,         \
-                           a.m.gather_entry, a.m.ghost, a.m.twin, a.dQL, a.dQ, cell0, ncell,    \
+                           a.m.gather_entry, a.dQL, a.dQ, cell0, ncell,                        \
                            qshift);                                                             \
         hipLaunchKernelGGL((ens::range_update<ND>), gc, b, 0, s, a.c, a.Q, a.dQ, a.m.volume,    \
                            a.W, a.cstatus, a.mass, a.ctr, cell0, ncell);                        \

@@ -278,7 +278,7 @@ __device__ __forceinline__ void q_faces(const EnsArgs<T>& a, const mixed::CF& cf
 template <int ND, int MIXED, typename T>
 __device__ __forceinline__ void q_gather(const EnsArgs<T>& a) {
     drain<false>(a.plan, 2, 0, [&](const Slot& sl, int64_t i) {
-        flux::gather_cell<ND, MIXED, T>(i, a.m.gather_off, a.m.gather_entry, a.m.ghost, a.m.twin,
+        flux::gather_cell<ND, MIXED, T>(i, a.m.gather_off, a.m.gather_entry,
                                         a.dQL, sl.qshift, a.dQ);
     });
 }

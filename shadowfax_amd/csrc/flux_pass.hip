@@ -72,7 +72,7 @@ hipError_t launch_face_fluxes<double>(int ndim, int kind, const flux::MeshView<d
     return hipGetLastError();
 }
 
-hipError_t launch_gather_fp64(int ndim, int64_t C, int64_t F, const int64_t* goff,
+hipError_t launch_gather_fp64(int ndim, int64_t C, const int64_t* goff,
                               const int32_t* gent, const double* dQL, double* dQ,
                               hipStream_t s) {
     if(C <= 0) return hipSuccess;

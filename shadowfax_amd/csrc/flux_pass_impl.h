@@ -1844,15 +1844,11 @@ __attribute__((amdgpu_waves_per_eu(face_waves<ND, KIND, MIXED, ROOT>(), 10))) vo
 template <int ND, int MIXED, typename T>
 __device__ __forceinline__ void gather_cell(int64_t i, const int64_t* __restrict__ goff,
                                             const int32_t* __restrict__ gent,
-                                            const uint8_t* __restrict__ ghost,
-                                            const int32_t* __restrict__ twin,
                                             const T* __restrict__ dQL, int64_t qshift,
                                             double* __restrict__ dQ) {
     const int NC = ND + 2;
     // every row of dQL holds its face's flux seen from the left cell (the
     // mixed face pass writes both copies of a periodic pair): no twins here
-    (void)ghost;
-    (void)twin;
     double acc[NC];
 #pragma unroll
     for(int k = 0; k < NC; k++) acc[k] = 0.0;

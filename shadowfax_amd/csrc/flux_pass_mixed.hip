@@ -109,9 +109,8 @@ hipError_t launch_face_records(int ndim, const flux::MeshView<float>& m, float* 
     return hipGetLastError();
 }
 
-hipError_t launch_gather_mixed(int ndim, int64_t C, int64_t F, const int64_t* goff,
-                               const int32_t* gent, const uint8_t* ghost, const int32_t* twin,
-                               const float* dQL, double* dQ, hipStream_t s) {
+hipError_t launch_gather_mixed(int ndim, int64_t C, const int64_t* goff,
+                               const int32_t* gent, const float* dQL, double* dQ, hipStream_t s) {
     if(C <= 0) return hipSuccess;
     flux::gather_shape<float>(ndim, [&](auto shape) {
         using S = decltype(shape);

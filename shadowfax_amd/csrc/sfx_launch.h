@@ -93,15 +93,14 @@ hipError_t launch_update(int ndim, const Consts& c, int64_t C, double* Q, double
                          const double* volume, double* W, const uint64_t* endtime,
                          uint64_t tnow, uint8_t* cstatus, double* mass,
                          unsigned long long* ctr, hipStream_t s);
-hipError_t launch_gather_fp64(int ndim, int64_t C, int64_t F, const int64_t* goff,
+hipError_t launch_gather_fp64(int ndim, int64_t C, const int64_t* goff,
                               const int32_t* gent, const double* dQL, double* dQ,
                               hipStream_t s);
 // flux_pass_mixed.hip: the mixed face kernel's per-face records (frec: 3 or
 // 4 float4 a face, m.F faces, see flux::face_record_kernel)
 hipError_t launch_face_records(int ndim, const flux::MeshView<float>& m, float* frec,
                                hipStream_t s);
-hipError_t launch_gather_mixed(int ndim, int64_t C, int64_t F, const int64_t* goff,
-                               const int32_t* gent, const uint8_t* ghost, const int32_t* twin,
-                               const float* dQL, double* dQ, hipStream_t s);
+hipError_t launch_gather_mixed(int ndim, int64_t C, const int64_t* goff,
+                               const int32_t* gent, const float* dQL, double* dQ, hipStream_t s);
 
 }  // namespace sfx

@@ -411,11 +411,10 @@ int sfx_gather_dQ(sfx_solver* h, const sfx_mesh* m, const void* dQL, double* dQ,
     if((rc = bind_device(h))) return rc;
     hipError_t e =
             (h->precision == SFX_PREC_FP64)
-                    ? launch_gather_fp64(h->ndim, m->C, m->F, m->gather_off, m->gather_entry,
+                    ? launch_gather_fp64(h->ndim, m->C, m->gather_off, m->gather_entry,
                                          (const double*)dQL, dQ, (hipStream_t)stream)
-                    : launch_gather_mixed(h->ndim, m->C, m->F, m->gather_off, m->gather_entry,
-                                          m->ghost, m->twin, (const float*)dQL, dQ,
-                                          (hipStream_t)stream);
+                    : launch_gather_mixed(h->ndim, m->C, m->gather_off, m->gather_entry,
+                                          (const float*)dQL, dQ, (hipStream_t)stream);
     if(e != hipSuccess) return hip_error(e, "gather kernel launch");
     return SFX_OK;
 }

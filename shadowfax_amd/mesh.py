@@ -407,7 +407,7 @@ class DeviceMesh:
         self.frec = None
         if self.face_records:
             planes = Cp.lib().sfx_mesh_face_record_planes(nd, Cp.SFX_PREC_MIXED)
-            self.frec = torch.zeros((planes, self.F, 4), dtype=torch.float32, device=self.dev)
+            self.frec = torch.zeros((planes * self.F, 4), dtype=torch.float32, device=self.dev)
         # the mixed gradients' closure correction, for face lists whose cells
         # do not close (None: they do)
         if storage == "mixed" and b.get("closure") is not None:
