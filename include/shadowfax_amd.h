@@ -98,12 +98,14 @@ int sfx_solver_enable_stats(sfx_solver* h, int enabled);
 /* Wave-level compaction of the mixed exact solver's batched path: every
  * problem gets `iterations` FP32 Newton iterations in the first kernel;
  * the ones still iterating (strong shocks, near vacuum) are queued with
- * their state and finished, densely packed, by a persistent second kernel,
- * so that a few slow lanes do not hold up their wavefront.  0 runs one
+ * their state, those beyond the FP32 iteration's range without any, and
+ * finished, densely packed, by a persistent second kernel, so that a few
+ * slow lanes do not hold up their wavefront.  0 runs one
  * kernel.  Results are identical either way.  Default 0: on MI355X the
- * bracketed FP32 Newton converges within a few steps even for the 1e6
- * shocks and near-vacuum faces, and no stop count from 1 to 24 made the
- * two kernels faster than one on the 4M-problem mixed batch.  (No
+ * FP32 Newton converges within a few steps even for the 1e6 shocks and
+ * near-vacuum faces, and no stop count from 1 to 24 made the two kernels
+ * faster than one on the 4M-problem mixed batch (100-106 us; 1: 198,
+ * 4: 114, 24: 100).  (No
  * reference counterpart: the reference solves one problem at a time.) */
 int sfx_solver_set_split(sfx_solver* h, int iterations);
 int sfx_solver_get_split(const sfx_solver* h);

@@ -16,7 +16,8 @@
 // Template parameters: ND (2, 3), KIND (0 exact, 1 HLLC), T (storage type of
 // cell states, gradients and face geometry) and R (arithmetic type of the
 // reconstruction).  The FP64 parity pass is T = R = double in a TU compiled
-// with -ffp-contract=off, every expression in the reference's association;
+// with -ffp-contract=off: gradients, sums and update in the reference's
+// association, the face's quotients rearranged (to round-off);
 // the mixed pass is T = float, R = double with the mixed Riemann solvers and
 // FP64 dQ.
 //

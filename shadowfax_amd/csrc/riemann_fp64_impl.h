@@ -1,10 +1,11 @@
 // riemann_fp64_impl.h -- FP64 device implementations of the exact and HLLC
-// Riemann solvers, following the reference expression by expression
-// (Shadowfax src/riemann/ExactRiemannSolver.cpp, HLLCRiemannSolver.cpp).
+// Riemann solvers (Shadowfax src/riemann/ExactRiemannSolver.cpp,
+// HLLCRiemannSolver.cpp): ex_solve_steps and hllc_steps expression by
+// expression, ex_solve and hllc_solve_for_flux the same iteration and formulas
+// over cheaper quotients, roots and powers, to round-off.
 // Included by riemann_fp64.hip and the flux-pass kernels, which are compiled
-// with -ffp-contract=off so the association (and rounding) of the reference
-// is kept, and by riemann_mixed.hip, whose HLLC path runs these functions on
-// FP32-stored inputs.
+// with -ffp-contract=off so that expressions keep their association, and by
+// riemann_mixed_impl.h for quotients and roots.
 #pragma once
 
 #include "sfx_device.h"

@@ -1,6 +1,6 @@
 """The mixed exact solver's iteration in the n-th root of p (gamma 5/3 and 7/5)
 over the range of states it takes -- densities and pressures to 1e28 and
-1e-28, pressure ratios on both sides of the limit (1e18), colliding and
+1e-28 and beyond, pressure ratios up to the limit (1e30), colliding and
 separating streams, equal states, walls -- against the FP64 solver on the same
 FP64-stored problems: 1e-6 normwise, the mixed path's contract."""
 import numpy as np
